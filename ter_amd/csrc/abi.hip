@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <queue>
 #include <new>
@@ -287,9 +288,7 @@ int pick_wg(long long total_tiles, int wg_per_cu, int lds_bytes, bool prologue, 
     return TER_HIP_OK;
 }
 
-// per_block: strips per block of the launch (kWaves * strips per wave for its row-block count).
-GemmDesc make_gemm_desc(const ter_hip_wpk_t* w, const int8_t* x, const float* xs, int M, const ter_hip_out_t& o,
-                        long long block0, int per_block, long long tile0) {
+GemmDesc make_gemm_desc(const ter_hip_wpk_t* w, const int8_t* x, const float* xs, int M, const ter_hip_out_t& o) {
     GemmDesc d{};
     d.w = w->data;
     d.x = x;
@@ -298,30 +297,109 @@ GemmDesc make_gemm_desc(const ter_hip_wpk_t* w, const int8_t* x, const float* xs
     d.acc = o.acc;
     d.y16 = o.y16;
     d.resid = o.resid;
-    d.block0 = block0;
-    d.tile0 = tile0;
     d.K = w->K;
     d.N = w->N;
     d.Ku = units_of(w->K);
     d.n_strips = strips_of(w->N);
     d.M = M;
     d.ldx = w->K;
-    d.n_blocks = (d.n_strips + per_block - 1) / per_block;
     d.w_scale = w->scale;
     d.w_mag = w->mag;
     return d;
 }
 
-bool gemm_vec_ok(const GemmDesc& d) { return aligned(d.x, 16) && d.ldx % 16 == 0; }
-
-// Rows per piece of the LDS-ring GEMM (8 row blocks).  A GEMM with more rows
-// (prefill) whose X rows are 16-byte aligned is cut into pieces of this many
-// rows over the same weights, so the ring kernel serves it instead of the
-// register-staged kernel (M = 256 on the BitNet-2B sweep: about 2x the
-// M = 128 time, against 11x).
+// Rows per piece of the LDS-ring GEMM (8 row blocks): a GEMM with more rows
+// (prefill) is cut into pieces of this many rows over the same weights.
 constexpr int kRingRows = 128;
+// Below this many bytes of X the split kernel reads it byte by byte.
+constexpr long long kSplitMinBytes = 16;
 
 bool ring_rows_ok(const int8_t* x, int K) { return aligned(x, 16) && K % 16 == 0; }
+
+// Latest finish when costs[i] are dealt out largest first to `slots`
+// workgroups, each to the one free first.
+double makespan(std::vector<double> costs, int slots) {
+    std::sort(costs.begin(), costs.end(), std::greater<double>());
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
+    double last = 0.0;
+    for (const double c : costs) {
+        double t = c;
+        if ((int)free_at.size() == slots) {
+            t += free_at.top();
+            free_at.pop();
+        }
+        free_at.push(t);
+        last = std::max(last, t);
+    }
+    return last;
+}
+
+// The kernel of a launch of `n` GEMMs (whole: not cut into row pieces): the
+// LDS-ring kernel or a tile of the split kernel, whichever takes less time by
+// two cost models.  The ring kernel needs 16-byte aligned X rows (vec) and
+// costs less per block, but its blocks are large and walk all of K: with few
+// of them most CUs idle (M = 128, K = N = 8192: 32 blocks, 44.6 us; split
+// 14.6), and in a short list the blocks with the longest K run last alone
+// (one BitNet layer's list, K = 2560 and 6912, at M = 128: 40 against 22 us).
+// Long lists are the ring kernel's (8 layers: 87 against 132 us).
+//
+// Split, one GEMM: its tiles take turns on the CUs (gemm_split_tile_us).  A
+// list: the longest tile, or the sum over the CUs times 1.4 (every CU reading
+// at once: at 8 layers and M = 128 the tiles cost 1.25-1.55 times their
+// single-GEMM time).  Ring: the list schedule's makespan, at a stage time
+// between that of few busy CUs and that of all (gemm_lds_unit_us).  Checked
+// for lists of 1-8 layers at M = 8-256 (BitNet-2B's shapes, and H = 768, F =
+// 2048 with up to 30 layers): the choice is the fastest of the seven, or
+// within 10% of it.
+struct GemmPick {
+    bool ring;
+    int tile;    // split kernel
+    bool longk;  // split kernel
+};
+GemmPick pick_gemm(const GemmDesc* whole, int n, int max_m, bool vec, int cus) {
+    GemmPick best{false, 0, false};
+    double best_us = 1e30;
+    int max_ku = 0;
+    for (int i = 0; i < n; ++i) max_ku = std::max(max_ku, whole[i].Ku);
+    best.longk = gemm_split_long(max_ku);
+    auto blocks_of = [&](int i, int rows, int strips) {
+        return (long long)((whole[i].M + rows - 1) / rows) * ((whole[i].n_strips + strips - 1) / strips);
+    };
+    for (int t = 0; t < gemm_split_tiles(); ++t) {
+        double us = 0.0, sum = 0.0;
+        for (int i = 0; i < n; ++i) {
+            const long long k = blocks_of(i, gemm_split_rows(t), gemm_split_strips(t));
+            const double c = gemm_split_tile_us(t, whole[i].Ku);
+            sum += (double)k * c;
+            us = std::max(us, n == 1 ? (double)((k + cus - 1) / cus) * c : c);
+        }
+        if (n > 1) us = std::max(us, 1.4 * sum / cus);
+        if (us < best_us) {
+            best_us = us;
+            best.tile = t;
+        }
+    }
+    if (!vec) return best;
+    const int mb = gemm_mb_of(std::min(max_m, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
+    std::vector<double> costs;
+    long long count = 0;
+    double sum = 0.0, last = 0.0;
+    for (int i = 0; i < n; ++i) {
+        const long long k = blocks_of(i, kRingRows, lbs);
+        count += k;
+        sum += (double)k * (whole[i].Ku + 1);
+    }
+    if (n == 1) {  // equal blocks
+        last = (double)((count + cus - 1) / cus) * (whole[0].Ku + 1);
+    } else if (count > 8LL * cus) {  // a long list packs evenly
+        last = sum / cus;
+    } else {
+        for (int i = 0; i < n; ++i) costs.insert(costs.end(), (size_t)blocks_of(i, kRingRows, lbs), whole[i].Ku + 1.0);
+        last = makespan(costs, cus);
+    }
+    best.ring = last * gemm_lds_unit_us(mb, std::min(1.0, sum / cus / last)) < best_us;
+    return best;
+}
 
 // The outputs of rows r0.. of an [M][N] output set.
 ter_hip_out_t out_rows(const ter_hip_out_t& o, int r0, int N) {
@@ -331,43 +409,12 @@ ter_hip_out_t out_rows(const ter_hip_out_t& o, int r0, int N) {
                          o.silu ? o.silu + off : nullptr};
 }
 
-// GEMM workgroups: up to kGemmWgPerCu per CU (more weight bytes in flight
-// for the HBM-bound small-M blocks), capped by occupancy and by the block count.
-constexpr int kGemmWgPerCu = 8;
-
-// Streaming GEMM (M <= 16): kGemmWgPerCuStream workgroups per CU, capped by
-// occupancy at this LDS size.
-constexpr int kGemmWgPerCuStream = 2;
-
-int pick_stream_wg(long long tiles, int lds, int wg_per_cu, int* n_wg) {
+int current_cu_count(int* cus) {
     int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    const hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    const int cus = device_cu_count(dev);
-    if (cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
-    const int fit = gemm_stream_max_wg_per_cu(lds);
-    if (fit <= 0) return fail(TER_HIP_ERR_HIP, "GEMM occupancy query failed");
-    const int per_cu = wg_per_cu > 0 ? wg_per_cu : (kGemmWgPerCuStream < fit ? kGemmWgPerCuStream : fit);
-    long long g = (long long)cus * per_cu;
-    if (g > tiles) g = tiles;
-    if (g < 1) g = 1;
-    *n_wg = (int)g;
-    return TER_HIP_OK;
-}
-
-int pick_gemm_wg(long long blocks, int mb, int wg_per_cu, int* n_wg) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    const int cus = device_cu_count(dev);
-    if (cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
-    const int fit = gemm_max_wg_per_cu(mb);
-    if (fit <= 0) return fail(TER_HIP_ERR_HIP, "GEMM occupancy query failed");
-    const int per_cu = wg_per_cu > 0 ? wg_per_cu : (kGemmWgPerCu < fit ? kGemmWgPerCu : fit);
-    long long g = (long long)cus * per_cu;
-    if (g > blocks) g = blocks;
-    if (g < 1) g = 1;
-    *n_wg = (int)g;
+    *cus = device_cu_count(dev);
+    if (*cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
     return TER_HIP_OK;
 }
 
@@ -403,13 +450,14 @@ struct ter_hip_plan {
     bool strided = false;        // GEMV strip mode: the strided RMS prologue (gemv_strided_ok for every item)
     bool shared = false;         // GEMV strided strip mode: one activation, back-to-back tile streams
     GemvDesc shared_desc{};      //   its kernel argument (shared_plan_desc)
-    int mb = 0;                  // GEMM row-block count
+    int mb = 0;                  // GEMM row-block count (LDS-ring kernel)
     bool vec = false;            // GEMM: 16-byte X rows
-    bool stream = false;         // GEMM: streaming kernel (M <= 16), total counts tiles
-
-    bool lds = false;            // GEMM: LDS-ring kernel (M <= 128 where streaming does not apply)
-    const GemmBlock* blocks_dev = nullptr;  // LDS-ring: [n_blocks] blocks, then
-    const int32_t* ranges_dev = nullptr;    //   [n_wg + 1] block ranges per workgroup
+    bool lds = false;            // GEMM: LDS-ring kernel, else the split kernel
+    int tile = 0;                //   the split kernel's tile, K split
+    bool longk = false;          //   (pick_gemm),
+    bool bytes_x = false;        //   and whether it reads X byte by byte
+    const GemmBlock* blocks_dev = nullptr;  // GEMM: [n_blocks] blocks, then
+    const int32_t* ranges_dev = nullptr;    //   (LDS-ring) [n_wg + 1] block ranges per workgroup
     const long long* wg_ranges_dev = nullptr;  // GEMV stream-K: [n_wg + 1] tile ranges per workgroup
     const void* wg_desc_dev = nullptr;         // GEMV strip mode: [n_wg] copies of each workgroup's first descriptor
     int n_blocks = 0;
@@ -636,8 +684,34 @@ static bool mm_row_stage(int dev, size_t xbytes, size_t ybytes, MmRowStage** out
     return true;
 }
 
-// Device copy of an LDS-ring GEMM plan: descriptors, the block list in
-// workgroup order, and the per-workgroup block ranges.  Range g holds
+// Device copy of a GEMM plan: descriptors, the block list, and (LDS-ring
+// kernel) the per-workgroup block ranges.
+int upload_blocks(ter_hip_plan* p, const std::vector<GemmDesc>& ds, const std::vector<GemmBlock>& blocks,
+                  const std::vector<int32_t>& ranges) {
+    const size_t db = sizeof(GemmDesc) * ds.size(), bb = sizeof(GemmBlock) * blocks.size();
+    hipError_t e = hipMalloc(&p->descs_dev, db + bb + sizeof(int32_t) * ranges.size());
+    if (e != hipSuccess) {
+        p->descs_dev = nullptr;
+        return hip_fail(e, "plan descriptor allocation");
+    }
+    char* base = static_cast<char*>(p->descs_dev);
+    e = hipMemcpy(base, ds.data(), db, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(base + db, blocks.data(), bb, hipMemcpyHostToDevice);
+    if (e == hipSuccess && !ranges.empty())
+        e = hipMemcpy(base + db + bb, ranges.data(), sizeof(int32_t) * ranges.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(p->descs_dev);
+        p->descs_dev = nullptr;
+        return hip_fail(e, "plan descriptor upload");
+    }
+    p->blocks_dev = reinterpret_cast<const GemmBlock*>(base + db);
+    p->ranges_dev = reinterpret_cast<const int32_t*>(base + db + bb);
+    p->n_blocks = (int)blocks.size();
+    return TER_HIP_OK;
+}
+
+// An LDS-ring GEMM plan: the block list in workgroup order and the
+// per-workgroup block ranges.  Range g holds
 // workgroup g's blocks in the order it runs them.  The blocks are dealt out
 // largest first, each to the workgroup that would be free first (list
 // scheduling; ties to the lowest workgroup).  The order is a stable sort by
@@ -650,7 +724,6 @@ static bool mm_row_stage(int dev, size_t xbytes, size_t ybytes, MmRowStage** out
 // for the epilogue.  Against contiguous ranges balanced by units (the
 // largest range 15% above the mean at 16 rows, 37% at 32 rows) this keeps
 // every range within about 5% of the mean.
-constexpr long long kRingMinBlocksPerCu = 4;
 int upload_lds_plan(ter_hip_plan* p, const std::vector<GemmDesc>& ds, const std::vector<GemmBlock>& blocks_in,
                     int bs, int n_wg) {
     const size_t nb = blocks_in.size();
@@ -682,26 +755,7 @@ int upload_lds_plan(ter_hip_plan* p, const std::vector<GemmDesc>& ds, const std:
         for (const int32_t b : per_wg[(size_t)g]) blocks.push_back(blocks_in[(size_t)b]);
     }
     ranges[(size_t)n_wg] = (int32_t)blocks.size();
-    const size_t db = sizeof(GemmDesc) * ds.size(), bb = sizeof(GemmBlock) * blocks.size();
-    hipError_t e = hipMalloc(&p->descs_dev, db + bb + sizeof(int32_t) * ranges.size());
-    if (e != hipSuccess) {
-        p->descs_dev = nullptr;
-        return hip_fail(e, "plan descriptor allocation");
-    }
-    char* base = static_cast<char*>(p->descs_dev);
-    e = hipMemcpy(base, ds.data(), db, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(base + db, blocks.data(), bb, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(base + db + bb, ranges.data(), sizeof(int32_t) * ranges.size(), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(p->descs_dev);
-        p->descs_dev = nullptr;
-        return hip_fail(e, "plan descriptor upload");
-    }
-    p->blocks_dev = reinterpret_cast<const GemmBlock*>(base + db);
-    p->ranges_dev = reinterpret_cast<const int32_t*>(base + db + bb);
-    p->n_blocks = (int)blocks.size();
-    return TER_HIP_OK;
+    return upload_blocks(p, ds, blocks, ranges);
 }
 
 extern "C" {
@@ -1153,14 +1207,10 @@ int ter_hip_plan_launch(const ter_hip_plan_t* plan, void* stream) {
         GemmDesc none{};
         e = launch_gemm_lds(none, static_cast<const GemmDesc*>(plan->descs_dev), plan->blocks_dev, plan->ranges_dev,
                             plan->n_blocks, plan->n_wg, plan->mb, static_cast<hipStream_t>(stream));
-    } else if (plan->gemm && plan->stream) {
-        GemmDesc none{};
-        e = launch_gemm_stream(none, static_cast<const GemmDesc*>(plan->descs_dev), plan->first_dev, plan->total,
-                               plan->n_wg, plan->lds_bytes, plan->vec, static_cast<hipStream_t>(stream));
     } else if (plan->gemm) {
         GemmDesc none{};
-        e = launch_gemm_list(none, static_cast<const GemmDesc*>(plan->descs_dev), plan->first_dev, plan->total,
-                             plan->n_wg, plan->mb, plan->vec, static_cast<hipStream_t>(stream));
+        e = launch_gemm_split(none, static_cast<const GemmDesc*>(plan->descs_dev), plan->blocks_dev, plan->n_blocks,
+                              plan->tile, plan->longk, plan->vec, plan->bytes_x, static_cast<hipStream_t>(stream));
     } else {
         GemvDesc none{};
         if (plan->strip_mode)
@@ -1280,13 +1330,18 @@ static int gemm_out_ws(const ter_hip_wpk_t* w, const ter_hip_act_t* x, int32_t M
         xq = q_ws;
         xs = s_ws;
     }
-    if (M > kRingRows && ring_rows_ok(xq, w->K)) {
+    const bool vec = ring_rows_ok(xq, w->K);
+    int cus = 0;
+    rc = current_cu_count(&cus);
+    if (rc) return rc;
+    const GemmDesc whole = make_gemm_desc(w, xq, xs, M, *out);
+    const GemmPick pick = pick_gemm(&whole, 1, M, vec, cus);
+    if (pick.ring) {
+        const int mb = gemm_mb_of(std::min(M, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
         // pieces of kRingRows rows, one LDS-ring launch each
-        const int mb = gemm_mb_of(kRingRows), lbs = gemm_lds_strips_per_block(mb);
         for (int r0 = 0; r0 < M; r0 += kRingRows) {
             const int m = std::min(kRingRows, M - r0);
-            const GemmDesc d = make_gemm_desc(w, xq + (size_t)r0 * w->K, xs + r0, m, out_rows(*out, r0, w->N), 0,
-                                              kWaves * gemm_strips_per_wave(mb), 0);
+            const GemmDesc d = make_gemm_desc(w, xq + (size_t)r0 * w->K, xs + r0, m, out_rows(*out, r0, w->N));
             const int nb = (d.n_strips + lbs - 1) / lbs;
             int n_wg = 0;
             rc = pick_lds_wg(nb, mb, &n_wg);
@@ -1296,27 +1351,8 @@ static int gemm_out_ws(const ter_hip_wpk_t* w, const ter_hip_act_t* x, int32_t M
         }
         return TER_HIP_OK;
     }
-    const int mb = gemm_mb_of(M);
-    const GemmDesc d = make_gemm_desc(w, xq, xs, M, *out, 0, kWaves * gemm_strips_per_wave(mb), 0);
-    int n_wg = 0;
-    hipError_t e;
-    const int slds = gemm_stream_lds_want(M, w->K);
-    const int lbs = gemm_vec_ok(d) ? gemm_lds_strips_per_block(mb) : 0;
-    if (gemm_stream_item_fits(M, w->K, slds)) {
-        const long long tiles = (long long)d.n_strips * d.Ku;
-        rc = pick_stream_wg(tiles, slds, 0, &n_wg);
-        if (rc) return rc;
-        e = launch_gemm_stream(d, nullptr, nullptr, tiles, n_wg, slds, gemm_vec_ok(d), st);
-    } else if (lbs > 0) {
-        const int nb = (d.n_strips + lbs - 1) / lbs;
-        rc = pick_lds_wg(nb, mb, &n_wg);
-        if (rc) return rc;
-        e = launch_gemm_lds(d, nullptr, nullptr, nullptr, nb, n_wg, mb, st);
-    } else {
-        rc = pick_gemm_wg(d.n_blocks, mb, 0, &n_wg);
-        if (rc) return rc;
-        e = launch_gemm_list(d, nullptr, nullptr, d.n_blocks, n_wg, mb, gemm_vec_ok(d), st);
-    }
+    const hipError_t e = launch_gemm_split(whole, nullptr, nullptr, 0, pick.tile, pick.longk, vec,
+                                           (long long)M * w->K < kSplitMinBytes, st);
     if (e != hipSuccess) return hip_fail(e, "gemm launch");
     return TER_HIP_OK;
 }
@@ -1348,15 +1384,12 @@ int ter_hip_gemm_out_static(const ter_hip_wpk_t* w, const ter_hip_act_t* x, int3
 }
 
 int ter_hip_gemm_plan_create(ter_hip_plan_t** plan, const ter_hip_gemm_item_t* items, int32_t n,
-                             int32_t wg_per_cu) {
+                             int32_t /* wg_per_cu: the kernels' own launch shapes */) {
     if (!plan || !items) return fail(TER_HIP_ERR_NULL, "null plan or items");
     *plan = nullptr;
     if (n < 1) return fail(TER_HIP_ERR_SHAPE, "empty work list");
-    std::vector<GemmDesc> ds((size_t)n);
-    long long blocks = 0;
     uint64_t bytes = 0, macs = 0;
     int max_m = 1;
-    bool vec = true;
     Ranges resid, inputs;
     for (int i = 0; i < n; ++i) {
         const ter_hip_gemm_item_t& it = items[i];
@@ -1375,92 +1408,76 @@ int ter_hip_gemm_plan_create(ter_hip_plan_t** plan, const ter_hip_gemm_item_t* i
         if (it.M > max_m) max_m = it.M;
     }
     if (int rc = check_resid_overlap(resid, inputs)) return rc;
-    // Items with more than kRingRows rows become pieces of kRingRows rows
-    // (one descriptor each) when every X qualifies for the LDS-ring kernel.
-    bool ring_all = true;
-    for (int i = 0; i < n; ++i) ring_all = ring_all && ring_rows_ok(items[i].x, items[i].w->K);
-    const int rows = max_m > kRingRows && ring_all ? kRingRows : TER_HIP_M_MAX;
-    const int mb = gemm_mb_of(std::min(max_m, rows));  // one row-block count (and block width) per launch
-    const int per_block = kWaves * gemm_strips_per_wave(mb);
-    long long tiles = 0;
-    ds.clear();
-    std::vector<long long> block_starts, tile_starts;
-    std::vector<int> piece0;  // first descriptor of each item (its pieces follow)
+    // One kernel, with one row-block count or tile, per launch.
+    bool vec = true, bytes_x = false;
+    for (int i = 0; i < n; ++i) {
+        vec = vec && ring_rows_ok(items[i].x, items[i].w->K);
+        bytes_x = bytes_x || (long long)items[i].M * items[i].w->K < kSplitMinBytes;
+    }
+    std::vector<GemmDesc> whole;
     for (int i = 0; i < n; ++i) {
         const ter_hip_gemm_item_t& it = items[i];
         const ter_hip_out_t o{it.y, it.acc, it.y16, it.resid, nullptr, nullptr};
-        piece0.push_back((int)ds.size());
-        for (int r0 = 0; r0 < it.M; r0 += rows) {
-            const int m = std::min(rows, it.M - r0);
-            const GemmDesc d = make_gemm_desc(it.w, it.x + (size_t)r0 * it.w->K, it.x_scale_dev + r0, m,
-                                              out_rows(o, r0, it.w->N), blocks, per_block, tiles);
-            ds.push_back(d);
-            block_starts.push_back(blocks);
-            tile_starts.push_back(tiles);
-            blocks += d.n_blocks;
-            tiles += (long long)d.n_strips * d.Ku;
-            vec = vec && gemm_vec_ok(d);
-        }
+        whole.push_back(make_gemm_desc(it.w, it.x, it.x_scale_dev, it.M, o));
         bytes += (uint64_t)it.w->K * (uint64_t)it.w->N / 4 + (uint64_t)it.M * it.w->K +
                  (uint64_t)it.M * it.w->N * out_bytes(o);
         macs += (uint64_t)it.M * (uint64_t)it.w->K * (uint64_t)it.w->N;
     }
-    n = (int)ds.size();
-    int n_wg = 0;
-    int slds = 0;  // the streaming kernel's LDS: the most any item wants
-    for (int i = 0; i < n; ++i) slds = std::max(slds, gemm_stream_lds_want(ds[(size_t)i].M, ds[(size_t)i].K));
-    bool stream = true;
-    for (int i = 0; i < n && stream; ++i) stream = gemm_stream_item_fits(ds[(size_t)i].M, ds[(size_t)i].K, slds);
-    // The LDS-ring kernel where the streamed one does not fit, and also
-    // where the list holds at least kRingMinBlocksPerCu of its blocks per CU:
-    // dealt out by list scheduling it beats the streamed kernel on large
-    // lists (C4 at 8 rows: 95.3 against 101.7 us; at 4 rows 88.7 against
-    // 95.5 us), while a short list needs the streamed kernel's split of K
-    // to fill the GPU (a ring block covers all of K for its strips).
-    int lbs = vec ? gemm_lds_strips_per_block(mb) : 0;
-    if (lbs > 0 && stream) {
-        long long ring_blocks = 0;
-        for (int i = 0; i < n; ++i) ring_blocks += (ds[(size_t)i].n_strips + lbs - 1) / lbs;
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return fail(TER_HIP_ERR_HIP, "hipGetDevice");
-        const int cus = device_cu_count(dev);
-        if (cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
-        if (ring_blocks < (long long)cus * kRingMinBlocksPerCu) lbs = 0;
-    }
-    ter_hip_plan* p = new (std::nothrow) ter_hip_plan();
-    if (!p) return fail(TER_HIP_ERR_ALLOC, "plan allocation");
-    int rc;
-    if (lbs > 0) {
-        // LDS-ring kernel: blocks of lbs strips, dealt out by list scheduling.
-        // The pieces of an item read the same weights: their blocks of one
-        // strip range are listed next to each other, so the scheduler hands
+    int cus = 0;
+    int rc = current_cu_count(&cus);
+    if (rc) return rc;
+    GemmPick pick = pick_gemm(whole.data(), n, max_m, vec, cus);
+    if (bytes_x) pick.tile = gemm_split_bytes_tile();
+    const bool ring = pick.ring && !bytes_x;
+    const int mb = gemm_mb_of(std::min(max_m, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
+    const int rows = ring ? kRingRows : gemm_split_rows(pick.tile), bs = ring ? lbs : gemm_split_strips(pick.tile);
+    std::vector<GemmDesc> ds;
+    std::vector<GemmBlock> bl;
+    for (int i = 0; i < n; ++i) {
+        const ter_hip_gemm_item_t& it = items[i];
+        const ter_hip_out_t o{it.y, it.acc, it.y16, it.resid, nullptr, nullptr};
+        const int d0 = (int)ds.size();
+        for (int r0 = 0; r0 < it.M; r0 += rows)
+            ds.push_back(make_gemm_desc(it.w, it.x + (size_t)r0 * it.w->K, it.x_scale_dev + r0,
+                                        std::min(rows, it.M - r0), out_rows(o, r0, it.w->N)));
+        // The pieces of an item read the same weights.  Ring: their blocks of
+        // one strip range are listed next to each other, so the scheduler hands
         // them out together to neighbouring workgroups on one XCD (equal cost,
         // adjacent in the stable order) and the pieces after the first find
         // the weight runs in that XCD's L2 instead of reading them again.
-        std::vector<GemmBlock> bl;
-        piece0.push_back(n);
-        for (size_t it = 0; it + 1 < piece0.size(); ++it) {
-            const int d0 = piece0[it], d1 = piece0[it + 1];
-            for (int st = 0; st < ds[(size_t)d0].n_strips; st += lbs)
-                for (int i = d0; i < d1; ++i) bl.push_back(GemmBlock{i, st});
-        }
+        // Split: one workgroup per block, in list order over the XCDs, so the
+        // pieces of a strip range sit 8 blocks apart.
+        const int group = ring ? bs : 8 * bs;
+        for (int s0 = 0; s0 < whole[(size_t)i].n_strips; s0 += group)
+            for (int p = d0; p < (int)ds.size(); ++p)
+                for (int st = s0; st < std::min(s0 + group, whole[(size_t)i].n_strips); st += bs)
+                    bl.push_back(GemmBlock{p, st});
+    }
+    n = (int)ds.size();
+    ter_hip_plan* p = new (std::nothrow) ter_hip_plan();
+    if (!p) return fail(TER_HIP_ERR_ALLOC, "plan allocation");
+    int n_wg = (int)bl.size();
+    if (ring) {
         rc = pick_lds_wg((long long)bl.size(), mb, &n_wg);
         if (!rc) rc = upload_lds_plan(p, ds, bl, lbs, n_wg);
     } else {
-        rc = stream ? pick_stream_wg(tiles, slds, wg_per_cu, &n_wg) : pick_gemm_wg(blocks, mb, wg_per_cu, &n_wg);
-        if (!rc) rc = stream ? upload_plan(p, ds, tile_starts, tiles, n_wg) : upload_plan(p, ds, block_starts, blocks, n_wg);
+        // the longest blocks first, so that none starts last
+        std::stable_sort(bl.begin(), bl.end(), [&](const GemmBlock& a, const GemmBlock& b) {
+            return ds[(size_t)a.desc].Ku > ds[(size_t)b.desc].Ku;
+        });
+        rc = upload_blocks(p, ds, bl, {});
     }
     if (rc) {
         delete p;
         return rc;
     }
-    p->lds = lbs > 0;
+    p->lds = ring;
+    p->tile = pick.tile;
+    p->longk = pick.longk;
+    p->bytes_x = bytes_x;
     p->n = n;
     p->gemm = true;
-    p->stream = stream;
-    p->total = stream ? tiles : blocks;
-    p->lds_bytes = stream ? slds : 0;
-
+    p->total = (long long)bl.size();
     p->n_wg = n_wg;
     p->mb = mb;
     p->vec = vec;

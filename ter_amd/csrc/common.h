@@ -29,8 +29,6 @@ namespace terhip {
 constexpr int kTileBytes = 1024;
 constexpr int kStripCols = 16;
 constexpr int kUnitK = 256;
-constexpr int kWaves = 4;                 // waves per workgroup of the GEMM kernels
-constexpr int kThreads = 64 * kWaves;
 constexpr int kGemvWaves = 4;             // waves per workgroup of the GEMV kernel
 constexpr int kGemvThreads = 64 * kGemvWaves;
 
@@ -68,8 +66,7 @@ struct alignas(16) GemvDesc {
     int32_t self;                // index of this descriptor in its plan's list (strip-mode plans)
 };
 
-// One GEMM (M > 1) of a work list.  Its blocks (4 column strips x all K each)
-// are numbered block0 .. block0 + n_blocks - 1 in the launch's block stream.
+// One GEMM (M > 1), or a piece of its rows, of a launch.
 struct alignas(16) GemmDesc {
     const uint8_t* w;            // T16 tile stream
     const int8_t* x;             // int8 [M][ldx]
@@ -78,10 +75,8 @@ struct alignas(16) GemmDesc {
     int32_t* acc;                // int32 [M][N] or null
     uint16_t* y16;               // fp16 [M][N] = half(y) or null
     float* resid;                // fp32 [M][N]: resid += float(half(y)), or null
-    long long block0;            // first block (unit-major kernel)
-    long long tile0;             // first tile in the launch's tile stream (streaming kernel)
     int32_t K, N, Ku, n_strips;
-    int32_t M, ldx, n_blocks;
+    int32_t M, ldx;
     float w_scale;
     int32_t w_mag;               // trit magnitude m of a {-m, 0, +m} payload (1 for plain trits)
 };
@@ -179,77 +174,37 @@ hipError_t launch_attn_decode(const uint16_t* q, const uint16_t* k, const uint16
 // Positions outside [0, smax) write nothing (both kernels).
 hipError_t launch_rope(uint16_t* v, int n_heads, int hd, const float* rope, const int32_t* pos, int smax, bool neox,
                        hipStream_t st);
-// Rows per MFMA row block group: MB = 1, 2, 4, 8, 16 for M up to 16, 32, 64, 128, 256.
-int gemm_mb_of(int M);
-// vec: every x pointer 16-byte aligned and every ldx a multiple of 16.
-hipError_t launch_gemm_list(const GemmDesc& single, const GemmDesc* list_dev, const int32_t* first_dev,
-                            long long total_blocks, int n_wg, int mb, bool vec, hipStream_t st);
-// Streaming GEMM for M <= 16 (whole X of a GEMM staged in LDS, whole strips
-// per wave, no per-unit barrier).  Each GEMM segment lays out the launch's
-// LDS for its own M and K: the X image, M rows of Ku * 16 chunks + one
-// padding chunk each (16 bytes per chunk), at [0, gemm_stream_zero_off); a
-// zero row of Ku * 256 bytes; 16 row sums; the waves' tile slots (each of the
-// 4 waves turns its tiles into MFMA operand order through two 1 KiB slots);
-// 16 row scales; then each wave's output buffer, as many whole strips as the
-// rest of the launch's LDS holds (up to kGemmStreamOutMax): the int32 results
-// of completed strips (M rows x 16 columns), written out between chunks of
-// the wave's tiles, so that no store is issued among the weight loads.  A
-// GEMM's X at K = 2560 leaves room for a whole run of strips (one write-out
-// per run); the stores cost about 10 us at M = 8 on the BitNet sweep
-// wherever they go, and 6 us more when split over five write-outs per run.
-__host__ __device__ inline int gemm_stream_zero_off(int M, int K) { return M * (units_of(K) * (kUnitK / 16) + 1) * 16; }
-constexpr int gemm_stream_slot_bytes() { return 4 * 2 * kTileBytes; }
-__host__ __device__ inline int gemm_stream_out_off(int M, int K) {
-    return gemm_stream_zero_off(M, K) + units_of(K) * kUnitK + 64 + gemm_stream_slot_bytes() + 64;
-}
-constexpr int kGemmStreamXMax = 64 * 1024;   // the X image (its staging registers hold 64 KiB)
-constexpr int kGemmStreamLdsMax = 80 * 1024; // in all: two workgroups per CU
-constexpr int kGemmStreamBatch = 6;          // tiles per batch (two batches per wave in flight)
-constexpr int kGemmStreamOutMax = 32;        // strips per output buffer at most
-// Strips of each wave's output buffer for a segment of this M and K in `lds` bytes.
-__host__ __device__ inline int gemm_stream_out_strips(int M, int K, int lds) {
-    const int left = lds - gemm_stream_out_off(M, K);
-    const int s = left > 0 ? left / (4 * M * kStripCols * 4) : 0;
-    return s < kGemmStreamOutMax ? s : kGemmStreamOutMax;
-}
-// A chunk is at least one double batch and completes at most
-// floor(chunk / Ku) + 1 strips, so a buffer needs floor(2 batch / Ku) + 1.
-__host__ __device__ inline int gemm_stream_out_need(int Ku) { return 2 * kGemmStreamBatch / Ku + 1; }
-// The LDS a GEMM of this M and K would take (full buffers), capped.
-inline int gemm_stream_lds_want(int M, int K) {
-    const int w = gemm_stream_out_off(M, K) + 4 * kGemmStreamOutMax * M * kStripCols * 4;
-    return w < kGemmStreamLdsMax ? w : kGemmStreamLdsMax;
-}
-// Whether a GEMM of this M and K streams in a launch of `lds` bytes.
-inline bool gemm_stream_item_fits(int M, int K, int lds) {
-    return M <= 16 && gemm_stream_zero_off(M, K) <= kGemmStreamXMax &&
-           gemm_stream_out_strips(M, K, lds) >= gemm_stream_out_need(units_of(K));
-}
-// lds_bytes: the launch's LDS (the largest gemm_stream_lds_want of the list).
-hipError_t launch_gemm_stream(const GemmDesc& single, const GemmDesc* list_dev, const int32_t* first_dev,
-                              long long total_tiles, int n_wg, int lds_bytes, bool vec, hipStream_t st);
-int gemm_stream_max_wg_per_cu(int lds_bytes);
-
-// Resident GEMM workgroups per CU for row-block count mb (0 if the query fails).
-int gemm_max_wg_per_cu(int mb);
-
-// LDS-ring GEMM for M <= 128 (mb = 1, 2, 4, 8; gemm_lds.hip), used where the
-// streaming kernel does not apply (M > 16, or M rows of X beyond its LDS).  Work is a
-// list of blocks, each `gemm_lds_strips_per_block(mb)` strips of one GEMM;
-// workgroup g (after the XCD remap) owns blocks [ranges[g], ranges[g+1]).
-// Single launches pass null lists and split n_blocks of `single` evenly.
-// Needs vec (16-byte aligned X rows).
 struct GemmBlock {
     int32_t desc;    // index into the descriptor list
     int32_t strip0;  // first strip of the block
 };
+// LDS-ring GEMM for M <= 128 (mb = 1, 2, 4, 8: row blocks of 16, gemm_mb_of;
+// gemm_lds.hip), for launches with enough blocks (pick_gemm in abi.hip).  Work is a
+// list of blocks, each `gemm_lds_strips_per_block(mb)` strips of one GEMM;
+// workgroup g (after the XCD remap) owns blocks [ranges[g], ranges[g+1]).
+// Single launches pass null lists and split n_blocks of `single` evenly.
+// Needs 16-byte aligned X rows.
+int gemm_mb_of(int M);
 int gemm_lds_strips_per_block(int mb);  // 0: no LDS-ring configuration for mb
+double gemm_lds_unit_us(int mb, double busy);
 int gemm_lds_max_wg_per_cu(int mb);
 hipError_t launch_gemm_lds(const GemmDesc& single, const GemmDesc* list_dev, const GemmBlock* blocks_dev,
                            const int32_t* ranges_dev, int n_blocks, int n_wg, int mb, hipStream_t st);
-// Column strips per wave of the GEMM for row-block count mb (a block is
-// kWaves * that many strips).
-int gemm_strips_per_wave(int mb);
+// Split GEMM (gemm_split.hip) for every other launch: a workgroup per tile of
+// gemm_split_rows x gemm_split_strips, any M, K and X alignment.  Lists take
+// one block per workgroup, each of a descriptor of at most gemm_split_rows
+// rows; single launches (null lists) cut `single` themselves.  longk: more
+// waves split K (gemm_split_long).  vec: every X row 16-byte aligned.  bytes:
+// some X is shorter than 16 bytes (all X read byte by byte, with the tile
+// gemm_split_bytes_tile).
+int gemm_split_tiles();
+int gemm_split_bytes_tile();
+int gemm_split_rows(int tile);
+int gemm_split_strips(int tile);
+float gemm_split_tile_us(int tile, int Ku);
+inline bool gemm_split_long(int Ku) { return Ku > 20; }
+hipError_t launch_gemm_split(const GemmDesc& single, const GemmDesc* list_dev, const GemmBlock* blocks_dev,
+                             int n_blocks, int tile, bool longk, bool vec, bool bytes, hipStream_t st);
 
 #if defined(__HIPCC__)
 #define TER_GLOBAL __attribute__((address_space(1)))

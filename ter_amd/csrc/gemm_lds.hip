@@ -1,7 +1,9 @@
 // gemm_lds.hip -- batched packed-trit GEMM for M <= 128 on gfx950 MFMA,
 // fed through an LDS ring by direct global->LDS loads.
 //
-// Same semantics as gemm.hip (cuda/ter_cuda_addonly_batched.cu:117-123):
+// Replaces the reference's batched kernels (mm_packed_batched,
+// cuda/ter_cuda_packed_batched.cu:26-83; mm_bitnet_addonly_batched_k<M>,
+// cuda/ter_cuda_addonly_batched.cu:31-124; the wmma s4 mm_int4_tc*):
 // acc[m][j] = sum_k X[m][k] w[k][j] in exact int32, y = float(mag * acc) * (xs[m] * w_scale).
 //
 // Work.  A block is BS consecutive column strips of one GEMM (all M rows,
@@ -806,6 +808,13 @@ int occupancy_cfg() {
 
 }  // namespace
 
+int gemm_mb_of(int M) {
+    if (M <= 16) return 1;
+    if (M <= 32) return 2;
+    if (M <= 64) return 4;
+    return 8;
+}
+
 int gemm_lds_strips_per_block(int mb) {
     switch (mb) {
         case 1: return Cfg1::BS;
@@ -814,6 +823,17 @@ int gemm_lds_strips_per_block(int mb) {
         case 8: return Cfg8::BS;
         default: return 0;
     }
+}
+
+// Time of a stage (one 256-row unit of a block) beyond a launch's fixed part,
+// with `busy` of the CUs at work, for the choice of the kernel (pick_gemm in
+// abi.hip): from single GEMMs of 16-32 blocks (K = N = 8192: 16.6, 37, 29 and
+// 45 us for 33 stages at M = 16, 32, 64 and 128) and from the BitNet-2B lists
+// at 30 layers (95, 115, 170 and 250 us for 136, 70, 136 and 136 stages per CU).
+double gemm_lds_unit_us(int mb, double busy) {
+    const double few = mb == 1 ? 0.40 : (mb == 2 ? 1.10 : (mb == 4 ? 0.91 : 1.40));
+    const double all = mb == 1 ? 0.70 : (mb == 2 ? 1.55 : (mb == 4 ? 1.25 : 1.80));
+    return few + (all - few) * busy;
 }
 
 int gemm_lds_max_wg_per_cu(int mb) {

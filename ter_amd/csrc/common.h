@@ -131,7 +131,7 @@ hipError_t launch_synth_v11(uint8_t* v11, int K, int N, uint64_t seed, uint32_t 
                             hipStream_t st);
 hipError_t launch_synth_i8(int8_t* x, long long n, uint64_t seed, int lo, int hi, hipStream_t st);
 hipError_t launch_quant_rows(const float* x, int M, int K, int8_t* q, float* s, hipStream_t st);
-// One workgroup of 256 threads per row; kind is TER_HIP_X_F32_RMS,
+// One workgroup per row; kind is TER_HIP_X_F32_RMS,
 // TER_HIP_X_F16_RMS or TER_HIP_X_RELU2_RMS (x = gate, up [M][K]).
 hipError_t launch_rmsnorm_quant_rows(const void* x, const uint16_t* up, int kind, const uint16_t* gamma, float eps,
                                      int M, int K, int8_t* q, float* s, hipStream_t st);

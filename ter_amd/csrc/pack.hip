@@ -141,93 +141,207 @@ __global__ void synth_i8_kernel(int8_t* __restrict__ x, long long n, uint64_t se
     x[i] = (int8_t)(lo + (int)((uu * span) >> 32));
 }
 
-// One workgroup (256 threads) per row: quant_int8_k steps
-// (cuda/ter_cuda_forward_packed.cu:40-62) on row m of x[M][K].
-__global__ __launch_bounds__(256) void quant_rows_kernel(const float* __restrict__ x, int K,
-                                                         int8_t* __restrict__ q,
-                                                         float* __restrict__ scale_out) {
+// Per-row quantizers, one workgroup per row: quant_int8_k
+// (cuda/ter_cuda_forward_packed.cu:40-62) alone (kind X_F32), or behind the
+// fused RMSNorm (rmsnorm_quant_f32_in_k / rmsnorm_quant_fp16_in_k,
+// cuda/ter_cuda_forward_bitnet.cu:64-146) or relu^2(gate) * up and RMSNorm
+// (relu2_mul_rmsnorm_quant_k, ibid.:258-309).  The sums of squares keep the
+// reference's order: 256 (relu^2: 1024) strided partials with fused
+// multiply-adds (the reference build contracts `local_sum += v * v`), then the
+// halving tree; rms_inv = 1 / sqrt(ss / K + eps) correctly rounded (the
+// reference's rsqrtf is an approximation); n = (x * rms_inv) * gamma.
+//
+// What bounds them: latency, with a workgroup per row and a row of a few KB.
+// A thread loads its NC chunks of 8 elements at once (16-byte loads where x,
+// up and gamma rows are 16-byte aligned with K a multiple of 8, else one load
+// per element), keeps them in registers through both passes, and the row is
+// read once.  For the norm's order the values also go to LDS as fp32, from
+// where the partials' threads read their strided elements; every wave then
+// forms the tree from the partials in LDS, so the sum needs two barriers and
+// the absmax one.  1024 threads past K = 4096 (a chunk or two each).  Before,
+// three passes of one-element loads: relu^2 at 64
+// rows of 6912 21.9 -> 3.9 us, fp32 RMSNorm at 64 rows of 2560 7.0 -> 3.0,
+// absmax at 256 rows of 2560 4.4 -> 2.6 (launches in a graph).
+template <int T, int NC, int KIND, bool kVec>
+__global__ __launch_bounds__(T) void quant_rows_kernel(const void* __restrict__ x, const uint16_t* __restrict__ up,
+                                                       const uint16_t* __restrict__ gamma, float eps, int K,
+                                                       int8_t* __restrict__ q, float* __restrict__ scale_out) {
 #pragma clang fp contract(off)
-    __shared__ float red[4];
-    const int m = blockIdx.x;
-    const float* xr = x + (long long)m * K;
-    float mx = 0.f;
-    for (int k = threadIdx.x; k < K; k += 256) mx = fmaxf(mx, fabsf(xr[k]));
-    mx = fmaxf(mx, __shfl_xor(mx, 1));
-    mx = fmaxf(mx, __shfl_xor(mx, 2));
-    mx = fmaxf(mx, __shfl_xor(mx, 4));
-    mx = fmaxf(mx, __shfl_xor(mx, 8));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float amax = mx + 1e-9f;
-    const float scale = 127.0f / amax;
-    if (threadIdx.x == 0) scale_out[m] = 1.0f / scale;
-    int8_t* qr = q + (long long)m * K;
-    for (int k = threadIdx.x; k < K; k += 256) {
-        const float v = xr[k] * scale;
-        int qi = (int)__builtin_rintf(v);
-        qi = qi > 127 ? 127 : (qi < -128 ? -128 : qi);
-        qr[k] = (int8_t)qi;
-    }
-}
-
-// One workgroup (256 threads) per row: the fused RMSNorm + int8 quantizer
-// (rmsnorm_quant_f32_in_k / rmsnorm_quant_fp16_in_k,
-// cuda/ter_cuda_forward_bitnet.cu:64-146) on row m of x[M][K]:
-// per-thread strided partial sums of squares with fused multiply-adds (the
-// reference build contracts `local_sum += v * v`), the reference's reduction
-// tree, rms_inv = 1 / sqrt(ss / K + eps) correctly rounded (the reference's
-// rsqrtf is an approximation), n = (x * rms_inv) * gamma, then quant_int8_k.
-// X_RELU2_RMS is relu2_mul_rmsnorm_quant_k (ibid.:258-309, one 1024-thread
-// block per row): x = relu^2(gate) * up and its 1024-strided sum order.
-__global__ __launch_bounds__(256) void rmsnorm_quant_rows_kernel(const void* __restrict__ x,
-                                                                 const uint16_t* __restrict__ up, int kind,
-                                                                 const uint16_t* __restrict__ gamma, float eps,
-                                                                 int K, int8_t* __restrict__ q,
-                                                                 float* __restrict__ scale_out) {
-#pragma clang fp contract(off)
-    __shared__ float red[256];
-    const int m = blockIdx.x, t = threadIdx.x;
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    constexpr bool kRms = KIND != TER_HIP_X_F32;
+    constexpr bool kF32 = KIND == TER_HIP_X_F32 || KIND == TER_HIP_X_F32_RMS;
+    constexpr int NP = KIND == TER_HIP_X_RELU2_RMS ? 1024 : 256;  // strided partial sums of squares
+    constexpr int EL = kF32 ? 4 : 2;
+    extern __shared__ __align__(16) float lds[];                  // kRms: the row's values [8 T NC], then partials [NP]
+    __shared__ float wmax[T / 64];
+    const int m = blockIdx.x, t = threadIdx.x, lane = t & 63;
     const long long row0 = (long long)m * K;
-    auto xv = [&](int k) -> float {
-        if (kind == TER_HIP_X_F32_RMS) return static_cast<const float*>(x)[row0 + k];
-        const float h = half_bits_to_float(static_cast<const uint16_t*>(x)[row0 + k]);
-        return kind == TER_HIP_X_F16_RMS ? h : relu2_mul(h, half_bits_to_float(up[row0 + k]));
-    };
-    float ss;
-    if (kind == TER_HIP_X_RELU2_RMS) {
-        ss = relu2_sum_sq_1024(static_cast<const uint16_t*>(x) + row0, up + row0, K, red);
-    } else {
-        float part = 0.f;
-        for (int k = t; k < K; k += 256) {
-            const float v = xv(k);
-            part = __builtin_fmaf(v, v, part);
-        }
-        ss = tree_sum256(part, red);
-    }
-    const float rms_inv = 1.0f / __builtin_sqrtf(ss / (float)K + eps);
-    float mx = 0.f;
-    for (int k = t; k < K; k += 256) {
-        const float n = (xv(k) * rms_inv) * half_bits_to_float(gamma[k]);
-        mx = fmaxf(mx, fabsf(n));
-    }
+    auto rsrc = [](const void* p, int bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000); };
+    const __amdgpu_buffer_rsrc_t xr = rsrc(static_cast<const char*>(x) + row0 * EL, K * EL);
+    const __amdgpu_buffer_rsrc_t ur = rsrc(up + row0, KIND == TER_HIP_X_RELU2_RMS ? 2 * K : 0);
+    const __amdgpu_buffer_rsrc_t gr = rsrc(gamma, kRms ? 2 * K : 0);
+
+    // element i of this thread's chunk c: 8 consecutive ones, or (one load per
+    // element) those a workgroup apart, so that a wave's loads stay contiguous
+    auto at = [t](int c, int i) { return kVec ? 8 * (t + T * c) + i : t + T * (8 * c + i); };
+    // raw values of every chunk (past K zeros), all loads issued first
+    auto load8 = [&](__amdgpu_buffer_rsrc_t r, int c, unsigned (&w)[4]) {  // 8 halves
+        if constexpr (kVec) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, 2 * at(c, 0), 0, 0);
+            w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+        } else {
 #pragma unroll
-    for (int s = 1; s < 64; s <<= 1) mx = fmaxf(mx, __shfl_xor(mx, s));
-    if ((t & 63) == 0) red[t >> 6] = mx;
+            for (int i = 0; i < 4; ++i)
+                w[i] = (unsigned)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * at(c, 2 * i), 0, 0) |
+                       (unsigned)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, 2 * at(c, 2 * i + 1), 0, 0) << 16;
+        }
+    };
+    unsigned xw[NC][kF32 ? 8 : 4], uw[NC][4], gw[NC][4];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if constexpr (kF32) {
+            if constexpr (kVec) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xr, 4 * at(c, 4 * h), 0, 0);
+                    xw[c][4 * h] = v.x; xw[c][4 * h + 1] = v.y; xw[c][4 * h + 2] = v.z; xw[c][4 * h + 3] = v.w;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) xw[c][i] = __builtin_amdgcn_raw_buffer_load_b32(xr, 4 * at(c, i), 0, 0);
+            }
+        } else {
+            load8(xr, c, xw[c]);
+        }
+        if constexpr (KIND == TER_HIP_X_RELU2_RMS) load8(ur, c, uw[c]);
+        if constexpr (kRms) load8(gr, c, gw[c]);
+    }
+    auto half_of = [](const unsigned (&w)[4], int i) { return half_bits_to_float((uint16_t)(w[i >> 1] >> (16 * (i & 1)))); };
+    float v[NC][8];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (kF32)
+                v[c][i] = __builtin_bit_cast(float, xw[c][i]);
+            else if constexpr (KIND == TER_HIP_X_F16_RMS)
+                v[c][i] = half_of(xw[c], i);
+            else
+                v[c][i] = relu2_mul(half_of(xw[c], i), half_of(uw[c], i));
+        }
+    if constexpr (kRms) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if constexpr (kVec) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    *reinterpret_cast<float4*>(lds + at(c, 4 * h)) =
+                        float4{v[c][4 * h], v[c][4 * h + 1], v[c][4 * h + 2], v[c][4 * h + 3]};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) lds[at(c, i)] = v[c][i];
+            }
+        }
+        __syncthreads();
+        // partial p: elements p, p + NP, .. in order (threads past NP idle; with
+        // fewer threads than partials each takes several)
+        float* part = lds + 8 * T * NC;
+        for (int p = t; p < NP; p += T) {
+            // (values past K are zeros: exact no-ops)
+            float s = 0.f;
+#pragma unroll 16
+            for (int i = 0; i < 8 * T * NC / NP; ++i) s = __builtin_fmaf(lds[p + NP * i], lds[p + NP * i], s);
+            part[p] = s;
+        }
+        __syncthreads();
+        // the tree's levels down to 64 per lane, then the wave's
+        auto p256 = [&](int i) {
+            if constexpr (NP == 1024)
+                return (part[i] + part[i + 512]) + (part[i + 256] + part[i + 768]);
+            else
+                return part[i];
+        };
+        const float ss = tree_down64((p256(lane) + p256(lane + 128)) + (p256(lane + 64) + p256(lane + 192)));
+        const float rms_inv = 1.0f / __builtin_sqrtf(ss / (float)K + eps);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[c][i] = (v[c][i] * rms_inv) * half_of(gw[c], i);
+    }
+    float mx = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (at(c, i) < K) mx = fmaxf(mx, fabsf(v[c][i]));
+    mx = fmaxf(mx, dpp_move_f<0xB1>(mx));   // lanes 1 and 2 apart (quad permutations), then the
+    mx = fmaxf(mx, dpp_move_f<0x4E>(mx));   // half-row and row mirrors, then across rows
+    mx = fmaxf(mx, dpp_move_f<0x141>(mx));
+    mx = fmaxf(mx, dpp_move_f<0x140>(mx));
+    mx = fmaxf(mx, lane_xor16(mx));
+    mx = fmaxf(mx, lane_xor32(mx));
+    if (lane == 0) wmax[t >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) mx = fmaxf(mx, wmax[w]);
     const float amax = mx + 1e-9f;
     const float scale = 127.0f / amax;
     if (t == 0) scale_out[m] = 1.0f / scale;
     int8_t* qr = q + row0;
-    for (int k = t; k < K; k += 256) {
-        const float n = (xv(k) * rms_inv) * half_bits_to_float(gamma[k]);
-        int qi = (int)__builtin_rintf(n * scale);
-        qi = qi > 127 ? 127 : (qi < -128 ? -128 : qi);
-        qr[k] = (int8_t)qi;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (at(c, 0) >= K) continue;
+        unsigned w[2] = {0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            int qi = (int)__builtin_rintf(v[c][i] * scale);
+            qi = qi > 127 ? 127 : (qi < -128 ? -128 : qi);
+            w[i >> 2] |= (unsigned)(uint8_t)qi << (8 * (i & 3));
+        }
+        if constexpr (kVec) {
+            *reinterpret_cast<TER_GLOBAL unsigned long long*>(gptr(qr) + at(c, 0)) =
+                (unsigned long long)w[0] | (unsigned long long)w[1] << 32;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (at(c, i) < K) gptr(qr)[at(c, i)] = (int8_t)(w[i >> 2] >> (8 * (i & 3)));
+        }
     }
+}
+
+template <int T, int NC, int KIND>
+hipError_t launch_quant_as(const void* x, const uint16_t* up, const uint16_t* gamma, float eps, int M, int K, int8_t* q,
+                           float* s, hipStream_t st) {
+    const int lds = KIND == TER_HIP_X_F32 ? 0 : (8 * T * NC + (KIND == TER_HIP_X_RELU2_RMS ? 1024 : 256)) * 4;
+    auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    const bool vec = K % 8 == 0 && a16(x) && a16(up) && a16(gamma) && (reinterpret_cast<uintptr_t>(q) & 7u) == 0;
+    // dynamic LDS above the 64 KiB default, once per instantiation
+    static const hipError_t allowed = [lds] {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, true>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, false>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        return e;
+    }();
+    if (allowed != hipSuccess) return allowed;
+    if (vec)
+        hipLaunchKernelGGL((quant_rows_kernel<T, NC, KIND, true>), dim3(M), dim3(T), lds, st, x, up, gamma, eps, K, q, s);
+    else
+        hipLaunchKernelGGL((quant_rows_kernel<T, NC, KIND, false>), dim3(M), dim3(T), lds, st, x, up, gamma, eps, K, q, s);
+    return hipGetLastError();
+}
+
+// Threads and chunks by K (at most 32768).
+template <int KIND>
+hipError_t launch_quant_kind(const void* x, const uint16_t* up, const uint16_t* gamma, float eps, int M, int K,
+                             int8_t* q, float* s, hipStream_t st) {
+    if (K <= 2048) return launch_quant_as<256, 1, KIND>(x, up, gamma, eps, M, K, q, s, st);
+    if (K <= 4096) return launch_quant_as<512, 1, KIND>(x, up, gamma, eps, M, K, q, s, st);
+    if (K <= 8192) return launch_quant_as<1024, 1, KIND>(x, up, gamma, eps, M, K, q, s, st);
+    if (K <= 16384) return launch_quant_as<1024, 2, KIND>(x, up, gamma, eps, M, K, q, s, st);
+    if (K <= 32768) return launch_quant_as<1024, 4, KIND>(x, up, gamma, eps, M, K, q, s, st);
+    return hipErrorInvalidValue;
 }
 
 inline unsigned grid_of(long long n, int block) { return (unsigned)((n + block - 1) / block); }
@@ -271,15 +385,14 @@ hipError_t launch_synth_i8(int8_t* x, long long n, uint64_t seed, int lo, int hi
 }
 
 hipError_t launch_rmsnorm_quant_rows(const void* x, const uint16_t* up, int kind, const uint16_t* gamma, float eps,
-                                     int M, int K,
-                                     int8_t* q, float* s, hipStream_t st) {
-    hipLaunchKernelGGL(rmsnorm_quant_rows_kernel, dim3(M), dim3(256), 0, st, x, up, kind, gamma, eps, K, q, s);
-    return hipGetLastError();
+                                     int M, int K, int8_t* q, float* s, hipStream_t st) {
+    if (kind == TER_HIP_X_F32_RMS) return launch_quant_kind<TER_HIP_X_F32_RMS>(x, nullptr, gamma, eps, M, K, q, s, st);
+    if (kind == TER_HIP_X_F16_RMS) return launch_quant_kind<TER_HIP_X_F16_RMS>(x, nullptr, gamma, eps, M, K, q, s, st);
+    return launch_quant_kind<TER_HIP_X_RELU2_RMS>(x, up, gamma, eps, M, K, q, s, st);
 }
 
 hipError_t launch_quant_rows(const float* x, int M, int K, int8_t* q, float* s, hipStream_t st) {
-    hipLaunchKernelGGL(quant_rows_kernel, dim3(M), dim3(256), 0, st, x, K, q, s);
-    return hipGetLastError();
+    return launch_quant_kind<TER_HIP_X_F32>(x, nullptr, nullptr, 0.f, M, K, q, s, st);
 }
 
 }  // namespace terhip

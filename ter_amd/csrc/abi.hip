@@ -793,10 +793,8 @@ int ter_hip_pack_v11(ter_hip_wpk_t* w, const uint8_t* v11_dev, void* stream) {
     if (!v11_dev) return fail(TER_HIP_ERR_NULL, "null v11 buffer");
     if (w->N % 4) return fail(TER_HIP_ERR_SHAPE, "v11 needs N %% 4 == 0 (N=%d)", w->N);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = launch_pack_v11(v11_dev, w->data, w->K, w->N, st);
+    hipError_t e = launch_pack_v11(v11_dev, w->data, w->fix, w->K, w->N, st);
     if (e != hipSuccess) return hip_fail(e, "pack_v11 launch");
-    e = hipMemsetAsync(w->fix, 0, (size_t)w->N * sizeof(uint64_t), st);
-    if (e != hipSuccess) return hip_fail(e, "fix-up slot clear");
     return TER_HIP_OK;
 }
 
@@ -808,10 +806,8 @@ int ter_hip_pack_i2s(ter_hip_wpk_t* w, const uint8_t* i2s_dev, void* stream) {
         return fail(TER_HIP_ERR_SHAPE, "i2_s needs K, N multiples of 4 and N*K a multiple of 128 (K=%d N=%d)", w->K,
                     w->N);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = launch_pack_i2s(i2s_dev, w->data, w->K, w->N, st);
+    hipError_t e = launch_pack_i2s(i2s_dev, w->data, w->fix, w->K, w->N, st);
     if (e != hipSuccess) return hip_fail(e, "pack_i2s launch");
-    e = hipMemsetAsync(w->fix, 0, (size_t)w->N * sizeof(uint64_t), st);
-    if (e != hipSuccess) return hip_fail(e, "fix-up slot clear");
     return TER_HIP_OK;
 }
 

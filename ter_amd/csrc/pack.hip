@@ -12,99 +12,147 @@
 namespace terhip {
 namespace {
 
-// 2-bit v11 code -> T16 field value u = w + 1 (code 11 decodes as 0 -> u = 1).
-__device__ __forceinline__ unsigned code_to_u(unsigned c) {
-    c &= 3u;
-    return c == 1u ? 2u : (c == 2u ? 0u : 1u);
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(1)));         // at any byte address
+typedef unsigned int u32_any __attribute__((aligned(1)));
+
+// Format conversion.  What bounds it: HBM, packed bytes in and packed bytes
+// out.  A thread makes one lane's 16 bytes of a T16 tile (4 columns x 16 rows
+// of K) from whole 16-byte pieces of the file format: v11 holds those 64
+// trits in 16 consecutive bytes of one column quad, i2_s in 16 consecutive
+// bytes of each column, and in both the four trits of a T16 field group come
+// out of one dword with a shift and a mask.  Measured at 6912 x 2560 (4.4 MB in
+// and out): i2_s 13.3 -> 4.3 us, v11 in 11.3 -> 3.5 us, v11 out 14.1 -> 3.6 us, against one byte load per
+// trit and one byte store per four.
+
+// Four 2-bit v11 codes, one per byte, -> u = w + 1 (00 -> 1, 01 -> 2, 10 -> 0, 11 -> 1).
+__device__ __forceinline__ unsigned codes_to_u(unsigned c) {
+    const unsigned k1 = 0x01010101u, b0 = c & k1, b1 = (c >> 1) & k1;
+    return ((b0 & ~b1) << 1) | (b0 ^ b1 ^ k1);
 }
 
-__device__ __forceinline__ unsigned u_to_code(unsigned u) {
-    return u == 2u ? 1u : (u == 0u ? 2u : 0u);
+// Four T16 fields u, one per byte, -> v11 codes (0 -> 10, 1 -> 00, 2 -> 01, 3 -> 00).
+__device__ __forceinline__ unsigned u_to_codes(unsigned u) {
+    const unsigned k1 = 0x01010101u, b0 = u & k1, b1 = (u >> 1) & k1;
+    return ((~(b0 | b1) & k1) << 1) | (b1 & ~b0);
 }
 
-// One thread per T16 dword: 16 trits of one column over 16 consecutive rows.
-__global__ void pack_v11_kernel(const uint8_t* __restrict__ v11, uint32_t* __restrict__ t16, int K,
-                                int N, int Ku, long long n_dwords) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_dwords) return;
-    const int j = (int)(i & 3);
-    const int lane = (int)((i >> 2) & 63);
-    const long long tile = i >> 8;
-    const int s = (int)(tile / Ku);
-    const int u = (int)(tile - (long long)s * Ku);
-    const int r = lane >> 4, q = lane & 15;
-    const int n = s * kStripCols + r * 4 + j;
-    const int k0 = u * kUnitK + q * 16;
-    unsigned out = 0;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int k = k0 + e;
-        unsigned uval = 1u;
-        if (n < N && k < K) uval = code_to_u(v11[(long long)(n >> 2) * K + k] >> (2 * (n & 3)));
-        const int f = e >> 2, b = e & 3;
-        out |= uval << (8 * b + 2 * f);
+// This thread's lane slot: tile (strip s, unit u), columns n0 .. n0 + 3 and
+// rows k0 .. k0 + 15 of K.
+struct LaneSlot {
+    int n0, k0, u, q;
+    __device__ LaneSlot(long long i, int Ku) {
+        const int lane = (int)(i & 63);
+        const long long tile = i >> 6;
+        const int s = (int)(tile / Ku);
+        u = (int)(tile - (long long)s * Ku);
+        q = lane & 15;
+        n0 = s * kStripCols + (lane >> 4) * 4;
+        k0 = u * kUnitK + q * 16;
     }
-    t16[i] = out;
+};
+
+// The fix-up slots of a strip's columns, zero at rest: written by its first
+// unit's threads (a fill inside the launch, where a memset would be a second
+// one and a memset node of a captured graph).
+__device__ __forceinline__ void clear_fix(const LaneSlot& l, unsigned long long* fix, int N) {
+    if (l.u == 0 && l.q < 4 && l.n0 + l.q < N) gptr(fix)[l.n0 + l.q] = 0ull;
 }
 
-// One thread per T16 dword, from microsoft/BitNet i2_s bytes
-// (tools/convert_bitnet_to_packed.py:85-157, vendor/ntransformer/core/dequant.cpp:114-145):
-// the (N, K) tensor row-major (element e = n K + k) in blocks of 128 elements
-// per 32 bytes; byte p of a block holds positions p, p+32, p+64, p+96 at
-// shifts 6, 4, 2, 0; codes 0 -> -1, 1 -> 0, 2 -> +1, 3 -> 0, i.e. u = w + 1 =
-// {0, 1, 2, 1}.  Padding rows / columns hold u = 1.
-__global__ void pack_i2s_kernel(const uint8_t* __restrict__ raw, uint32_t* __restrict__ t16, int K, int N,
-                                int Ku, long long n_dwords) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_dwords) return;
-    const int j = (int)(i & 3);
-    const int lane = (int)((i >> 2) & 63);
-    const long long tile = i >> 8;
-    const int s = (int)(tile / Ku);
-    const int u = (int)(tile - (long long)s * Ku);
-    const int r = lane >> 4, q = lane & 15;
-    const int n = s * kStripCols + r * 4 + j;
-    const int k0 = u * kUnitK + q * 16;
-    unsigned out = 0;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int k = k0 + e;
-        unsigned uval = 1u;
-        if (n < N && k < K) {
-            const long long el = (long long)n * K + k;
-            const long long blk = el >> 7;
-            const int pos = (int)(el & 127);
-            const unsigned code = (raw[blk * 32 + (pos & 31)] >> (6 - 2 * (pos >> 5))) & 3u;
-            uval = code == 3u ? 1u : code;  // w + 1 for w = {-1, 0, +1, 0}
+__global__ __launch_bounds__(256) void pack_v11_kernel(const uint8_t* __restrict__ v11, u32x4* __restrict__ t16,
+                                                       unsigned long long* __restrict__ fix, int K, int N, int Ku,
+                                                       long long n_slots) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_slots) return;
+    const LaneSlot l(i, Ku);
+    clear_fix(l, fix, N);
+    u32x4 raw = {0u, 0u, 0u, 0u};  // (code 00 is w = 0, the padding)
+    if (l.n0 < N && l.k0 < K) {
+        const TER_GLOBAL uint8_t* p = gptr(v11) + (long long)(l.n0 >> 2) * K + l.k0;
+        if (l.k0 + 16 <= K) {
+            raw = *reinterpret_cast<const TER_GLOBAL u32x4_any*>(p);
+        } else {
+            for (int e = 0; e < K - l.k0; ++e) raw[e >> 2] |= (unsigned)p[e] << (8 * (e & 3));
         }
-        const int f = e >> 2, b = e & 3;
-        out |= uval << (8 * b + 2 * f);
+    }
+    u32x4 out;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        unsigned d = 0;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) d |= codes_to_u((raw[f] >> (2 * j)) & 0x03030303u) << (2 * f);
+        out[j] = d;
     }
     t16[i] = out;
 }
 
-// One thread per v11 byte.
-__global__ void unpack_v11_kernel(const uint32_t* __restrict__ t16, uint8_t* __restrict__ v11, int K,
-                                  int N, int Ku) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)(N / 4) * K;
-    if (i >= total) return;
-    const int jb = (int)(i / K);
-    const int k = (int)(i - (long long)jb * K);
-    const int u = k / kUnitK;
-    const int q = (k % kUnitK) / 16;
-    const int e = k & 15;
-    const int f = e >> 2, b = e & 3;
-    unsigned byte = 0;
+// From microsoft/BitNet i2_s bytes (tools/convert_bitnet_to_packed.py:85-157,
+// vendor/ntransformer/core/dequant.cpp:114-145): the (N, K) tensor row-major
+// (element e = n K + k) in blocks of 128 elements per 32 bytes; byte p of a
+// block holds positions p, p+32, p+64, p+96 at shifts 6, 4, 2, 0; codes 0 -> -1,
+// 1 -> 0, 2 -> +1, 3 -> 0, i.e. u = w + 1 = {0, 1, 2, 1}.  K is a multiple of 4,
+// so four rows of K lie in one dword of the codes at one shift; with K a
+// multiple of 16 (k16) a thread's 16 rows lie in 16 consecutive bytes.
+template <bool k16>
+__global__ __launch_bounds__(256) void pack_i2s_kernel(const uint8_t* __restrict__ raw, u32x4* __restrict__ t16,
+                                                       unsigned long long* __restrict__ fix, int K, int N, int Ku,
+                                                       long long n_slots) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_slots) return;
+    const LaneSlot l(i, Ku);
+    clear_fix(l, fix, N);
+    const unsigned kM = 0x03030303u, k1 = 0x01010101u;
+    u32x4 out;
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub) {
-        const int n = jb * 4 + sub;
-        const int s = n / kStripCols, r = (n % kStripCols) / 4, j = n & 3;
-        const long long dw = (((long long)s * Ku + u) * 64 + (r * 16 + q)) * 4 + j;
-        const unsigned uval = (t16[dw] >> (8 * b + 2 * f)) & 3u;
-        byte |= u_to_code(uval) << (2 * sub);
+    for (int j = 0; j < 4; ++j) {
+        out[j] = 0x55555555u;  // u = 1: w = 0
+        if (l.n0 + j >= N || l.k0 >= K) continue;
+        const long long el = (long long)(l.n0 + j) * K + l.k0;
+        u32x4 w;
+        if constexpr (k16)
+            w = *reinterpret_cast<const TER_GLOBAL u32x4_any*>(gptr(raw) + (el >> 7) * 32 + (el & 31));
+        unsigned d = 0;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const long long ef = el + 4 * f;
+            unsigned c = 0;
+            if constexpr (k16) {
+                c = w[f];
+            } else if (l.k0 + 4 * f < K) {
+                c = *reinterpret_cast<const TER_GLOBAL u32_any*>(gptr(raw) + (ef >> 7) * 32 + (ef & 31));
+            } else {
+                c = 0x55555555u;  // code 1
+            }
+            c = (c >> (6 - 2 * (int)((ef & 127) >> 5))) & kM;
+            c ^= (c & (c >> 1) & k1) << 1;  // code 3 -> 1
+            d |= c << (2 * f);
+        }
+        out[j] = d;
     }
-    v11[i] = (uint8_t)byte;
+    t16[i] = out;
+}
+
+__global__ __launch_bounds__(256) void unpack_v11_kernel(const u32x4* __restrict__ t16, uint8_t* __restrict__ v11,
+                                                         int K, int N, int Ku, long long n_slots) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_slots) return;
+    const LaneSlot l(i, Ku);
+    if (l.n0 >= N || l.k0 >= K) return;
+    const u32x4 w = t16[i];
+    u32x4 out;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        unsigned d = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d |= u_to_codes((w[j] >> (2 * f)) & 0x03030303u) << (2 * j);
+        out[f] = d;
+    }
+    TER_GLOBAL uint8_t* p = gptr(v11) + (long long)(l.n0 >> 2) * K + l.k0;
+    if (l.k0 + 16 <= K) {
+        *reinterpret_cast<TER_GLOBAL u32x4_any*>(p) = out;
+    } else {
+        for (int e = 0; e < K - l.k0; ++e) p[e] = (uint8_t)(out[e >> 2] >> (8 * (e & 3)));
+    }
 }
 
 __device__ __forceinline__ uint64_t splitmix(uint64_t seed, uint64_t idx) {
@@ -167,7 +215,6 @@ __global__ __launch_bounds__(T) void quant_rows_kernel(const void* __restrict__ 
                                                        const uint16_t* __restrict__ gamma, float eps, int K,
                                                        int8_t* __restrict__ q, float* __restrict__ scale_out) {
 #pragma clang fp contract(off)
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     constexpr bool kRms = KIND != TER_HIP_X_F32;
     constexpr bool kF32 = KIND == TER_HIP_X_F32 || KIND == TER_HIP_X_F32_RMS;
     constexpr int NP = KIND == TER_HIP_X_RELU2_RMS ? 1024 : 256;  // strided partial sums of squares
@@ -348,26 +395,32 @@ inline unsigned grid_of(long long n, int block) { return (unsigned)((n + block -
 
 }  // namespace
 
-hipError_t launch_pack_v11(const uint8_t* v11, uint8_t* t16, int K, int N, hipStream_t st) {
+hipError_t launch_pack_v11(const uint8_t* v11, uint8_t* t16, uint64_t* fix, int K, int N, hipStream_t st) {
     const int Ku = units_of(K);
-    const long long n_dwords = (long long)strips_of(N) * Ku * (kTileBytes / 4);
-    hipLaunchKernelGGL(pack_v11_kernel, dim3(grid_of(n_dwords, 256)), dim3(256), 0, st, v11,
-                       reinterpret_cast<uint32_t*>(t16), K, N, Ku, n_dwords);
+    const long long n = (long long)strips_of(N) * Ku * 64;
+    hipLaunchKernelGGL(pack_v11_kernel, dim3(grid_of(n, 256)), dim3(256), 0, st, v11, reinterpret_cast<u32x4*>(t16),
+                       reinterpret_cast<unsigned long long*>(fix), K, N, Ku, n);
     return hipGetLastError();
 }
 
-hipError_t launch_pack_i2s(const uint8_t* raw, uint8_t* t16, int K, int N, hipStream_t st) {
+hipError_t launch_pack_i2s(const uint8_t* raw, uint8_t* t16, uint64_t* fix, int K, int N, hipStream_t st) {
     const int Ku = units_of(K);
-    const long long n_dwords = (long long)strips_of(N) * Ku * (kTileBytes / 4);
-    hipLaunchKernelGGL(pack_i2s_kernel, dim3(grid_of(n_dwords, 256)), dim3(256), 0, st, raw,
-                       reinterpret_cast<uint32_t*>(t16), K, N, Ku, n_dwords);
+    const long long n = (long long)strips_of(N) * Ku * 64;
+    auto* f = reinterpret_cast<unsigned long long*>(fix);
+    if (K % 16 == 0)
+        hipLaunchKernelGGL(pack_i2s_kernel<true>, dim3(grid_of(n, 256)), dim3(256), 0, st, raw,
+                           reinterpret_cast<u32x4*>(t16), f, K, N, Ku, n);
+    else
+        hipLaunchKernelGGL(pack_i2s_kernel<false>, dim3(grid_of(n, 256)), dim3(256), 0, st, raw,
+                           reinterpret_cast<u32x4*>(t16), f, K, N, Ku, n);
     return hipGetLastError();
 }
 
 hipError_t launch_unpack_v11(const uint8_t* t16, uint8_t* v11, int K, int N, hipStream_t st) {
-    const long long total = (long long)(N / 4) * K;
-    hipLaunchKernelGGL(unpack_v11_kernel, dim3(grid_of(total, 256)), dim3(256), 0, st,
-                       reinterpret_cast<const uint32_t*>(t16), v11, K, N, units_of(K));
+    const int Ku = units_of(K);
+    const long long n = (long long)strips_of(N) * Ku * 64;
+    hipLaunchKernelGGL(unpack_v11_kernel, dim3(grid_of(n, 256)), dim3(256), 0, st,
+                       reinterpret_cast<const u32x4*>(t16), v11, K, N, Ku, n);
     return hipGetLastError();
 }
 

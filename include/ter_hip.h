@@ -240,8 +240,9 @@ int ter_hip_mm_packed_dispatch_f16(const int8_t* X, const float* scale_x_dev,
  * The library narrows the row into its own page-locked host buffer and the
  * GEMV writes its outputs into another (one pair per device, grown on demand
  * and held until the process ends; calls are serialized on them), so a call
- * is one upload, one kernel and one synchronize; `y_stage_dev` (N fp32) is
- * used only where page-locked memory cannot be had (pageable copies). */
+ * is one upload, the GEMV, and a wait for a number that the stream writes to
+ * host memory behind it; `y_stage_dev` (N fp32) is used only where page-locked
+ * memory cannot be had (pageable copies). */
 int ter_hip_mm_row(const int32_t* X, int32_t row, int32_t K, float x_scale,
                    const ter_hip_wpk_t* W, int32_t N, float* out,
                    void* x_stage_dev, float* y_stage_dev, void* stream);

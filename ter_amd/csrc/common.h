@@ -478,6 +478,8 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int hip_fail(hipError_t e, const char* what);
 
 int device_cu_count(int device);
+// Resident workgroups per CU of a kernel at this LDS size (0 if the query fails).
+int max_blocks_per_cu(const void* fn, int threads, int lds_bytes);
 // Resident GEMV workgroups per CU at this LDS size (0 if the query fails).
 int gemv_max_wg_per_cu(int lds_bytes, int vec_kind = -1);
 

@@ -800,10 +800,7 @@ hipError_t launch_cfg(const GemmDesc& single, const GemmDesc* list, const GemmBl
 template <class C>
 int occupancy_cfg() {
     if (allow_lds<C>() != hipSuccess) return 0;
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemm_lds_kernel<C, true>, C::THREADS, C::LDS) != hipSuccess)
-        return 0;
-    return n;
+    return max_blocks_per_cu(reinterpret_cast<const void*>(&gemm_lds_kernel<C, true>), C::THREADS, C::LDS);
 }
 
 }  // namespace

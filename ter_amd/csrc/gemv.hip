@@ -1696,21 +1696,11 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
 }  // namespace
 
 int gemv_max_wg_per_cu(int lds_bytes, int vec_kind) {
-    int n = 0;
-    hipError_t e;
-    switch (vec_kind) {
-    case TER_HIP_X_I8:
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemv_t16_kernel<true, TER_HIP_X_I8>, kGemvThreads,
-                                                         lds_bytes);
-        break;
-    case TER_HIP_X_F32:
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemv_t16_kernel<true, TER_HIP_X_F32>, kGemvThreads,
-                                                         lds_bytes);
-        break;
-    default:  // the general kernel needs the most registers of all
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemv_t16_kernel<true, -1>, kGemvThreads, lds_bytes);
-    }
-    return e == hipSuccess ? n : 0;
+    // (by default the general kernel, which needs the most registers of all)
+    const void* fn = reinterpret_cast<const void*>(&gemv_t16_kernel<true, -1>);
+    if (vec_kind == TER_HIP_X_I8) fn = reinterpret_cast<const void*>(&gemv_t16_kernel<true, TER_HIP_X_I8>);
+    if (vec_kind == TER_HIP_X_F32) fn = reinterpret_cast<const void*>(&gemv_t16_kernel<true, TER_HIP_X_F32>);
+    return max_blocks_per_cu(fn, kGemvThreads, lds_bytes);
 }
 
 hipError_t launch_gemv(const GemvDesc& single, const GemvDesc* list_dev, const int32_t* first_dev,

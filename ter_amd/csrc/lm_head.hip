@@ -554,11 +554,8 @@ LmKernel lm_kernel_of(int H) {
 int lm_head_max_wg_per_cu(int H) {
     const int lds = lm_head_lds_bytes(H, 2048);
     const LmKernel k = lm_kernel_of(H);
-    int n = 0;
-    const hipError_t e =
-        k ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kLmThreads, lds)
-          : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, lm_head_generic_kernel, kLmThreads, lds);
-    return e == hipSuccess ? n : 0;
+    return max_blocks_per_cu(k ? reinterpret_cast<const void*>(k) : reinterpret_cast<const void*>(&lm_head_generic_kernel),
+                             kLmThreads, lds);
 }
 
 hipError_t launch_lm_head(const float* hidden, const uint16_t* hidden16, const uint16_t* gamma, float eps,

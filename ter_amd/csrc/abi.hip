@@ -231,18 +231,20 @@ constexpr long long kMaxPieceTiles = 1 << 20;
 // gamma 16-byte aligned; the staged kinds' fp32 staging fits), else -1 (the
 // general prologue).  X_F16 and X_SILU_MUL have a vector prologue only in
 // strip mode (strided); elsewhere their kind launches the general kernel.
-int gemv_vec_kind(const ter_hip_gemv_item_t* items, int n) {
+int act_vec_kind(const ter_hip_act_t& x, int K) {
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    const int kind = items[0].x.kind;
-    for (int i = 0; i < n; ++i) {
-        const ter_hip_act_t& x = items[i].x;
-        if (x.kind != kind || items[i].w->K % 16 != 0 || !a16(x.data)) return -1;
-        if (x.kind == TER_HIP_X_I16) return -1;  // the general prologue
-        if (stages32(x.kind) && !gemv_stage32(items[i].w->K)) return -1;  // the vector prologues always stage
-        if (gated(x.kind) && !a16(x.up)) return -1;
-        if (is_rms(x.kind) && !a16(x.gamma)) return -1;
-    }
-    return kind;
+    if (K % 16 != 0 || !a16(x.data)) return -1;
+    if (x.kind == TER_HIP_X_I16) return -1;  // the general prologue
+    if (stages32(x.kind) && !gemv_stage32(K)) return -1;  // the vector prologues always stage
+    if (gated(x.kind) && !a16(x.up)) return -1;
+    if (is_rms(x.kind) && !a16(x.gamma)) return -1;
+    return x.kind;
+}
+
+int gemv_vec_kind(const ter_hip_gemv_item_t* items, int n) {
+    for (int i = 0; i < n; ++i)
+        if (items[i].x.kind != items[0].x.kind || act_vec_kind(items[i].x, items[i].w->K) < 0) return -1;
+    return items[0].x.kind;
 }
 
 // Strip mode for work lists below kSmallPlanTilesPerWg tiles per workgroup at
@@ -824,6 +826,42 @@ int upload_lds_plan(ter_hip_plan* p, const std::vector<GemmDesc>& ds, const std:
     return upload_blocks(p, ds, blocks, ranges);
 }
 
+// One GEMM on int8 rows.
+static int run_gemm(const GemmDesc& whole, const ter_hip_out_t& out, hipStream_t st) {
+    const int M = whole.M;
+    const bool vec = ring_rows_ok(whole.x, whole.K);
+    int cus = 0;
+    int rc = current_cu_count(&cus);
+    if (rc) return rc;
+    const GemmPick pick = pick_gemm(&whole, 1, M, vec && whole.xs, cus);  // (the ring kernel reads device scales)
+    if (pick.ring) {
+        const int mb = gemm_mb_of(std::min(M, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
+        // pieces of kRingRows rows, one LDS-ring launch each
+        for (int r0 = 0; r0 < M; r0 += kRingRows) {
+            const ter_hip_out_t o = out_rows(out, r0, whole.N);
+            GemmDesc d = whole;
+            d.x += (size_t)r0 * whole.K;
+            d.xs += r0;
+            d.M = std::min(kRingRows, M - r0);
+            d.y = o.y;
+            d.acc = o.acc;
+            d.y16 = o.y16;
+            d.resid = o.resid;
+            const int nb = (d.n_strips + lbs - 1) / lbs;
+            int n_wg = 0;
+            rc = pick_lds_wg(nb, mb, &n_wg);
+            if (rc) return rc;
+            const hipError_t e = launch_gemm_lds(d, nullptr, nullptr, nullptr, nb, n_wg, mb, st);
+            if (e != hipSuccess) return hip_fail(e, "gemm launch");
+        }
+        return TER_HIP_OK;
+    }
+    const hipError_t e = launch_gemm_split(whole, nullptr, nullptr, 0, pick.tile, pick.longk, vec,
+                                           (long long)M * whole.K < kSplitMinBytes, st);
+    if (e != hipSuccess) return hip_fail(e, "gemm launch");
+    return TER_HIP_OK;
+}
+
 extern "C" {
 
 const char* ter_hip_version(void) { return "ter_hip 0.1.0 (gfx950, T16 layout)"; }
@@ -961,31 +999,54 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
         rc = check_resid_overlap(rr, in);
         if (rc) return rc;
     }
+    const long long total = (long long)strips_of(w->N) * units_of(w->K);
+    int cus = 0;
+    rc = current_cu_count(&cus);
+    if (rc) return rc;
+    if (x->kind == TER_HIP_X_I8 && !out->resid16 && !out->silu &&
+        (x->scale_dev || total < (long long)cus * kGemvWgPerCu * kSmallPlanTilesPerWg)) {
+        // int8 X needs no prologue: the GEMM kernels at M = 1 (fifteen of an
+        // MFMA's sixteen rows are padding, but these launches are bound by
+        // latency and HBM; in graphs: 2560 x 640 3.4 against 4.5 us, 6912 x 2560
+        // 4.4 against 6.0, 2048 x 128256 13.4 against 16.1, unaligned 1003 x
+        // 1236 3.4 against 5.1).  With a host scale the ring kernel is out
+        // (it loads device scales), and past strip mode's size the stream-K
+        // kernel takes over from the split one.
+        GemmDesc gd = make_gemm_desc(w, static_cast<const int8_t*>(x->data), x->scale_dev, 1, *out);
+        gd.x_scale = x->scale;
+        return run_gemm(gd, *out, static_cast<hipStream_t>(stream));
+    }
     const GemvDesc d = make_desc(w, x, *out, 0);
     if (x->kind == TER_HIP_X_I16) return launch_x16(d, static_cast<hipStream_t>(stream));
-    const long long total = (long long)d.n_strips * d.Ku;
     int n_wg = 0;
     const bool prologue = x->kind != TER_HIP_X_I8;
-    // small GEMVs: strip mode, as for a plan (whole strips per workgroup,
-    // the waves' partials added in LDS, no fix-up slots)
+    // as for a plan: the prologue of the activation's kind where its alignment
+    // allows (in graphs, 2560 x 640: fp32 RMSNorm 7.4 -> 4.7 us, relu^2 7.5 ->
+    // 5.6, fp16 absmax 5.9 -> 3.9 against the general one), and strip mode for
+    // small GEMVs (whole strips per workgroup, the waves' partials added in
+    // LDS, no fix-up slots)
+    const int vec_kind = act_vec_kind(*x, w->K);
     bool strip_mode = false;
     rc = pick_strip_mode(total, d.n_strips, prologue, &strip_mode, &n_wg);
     if (rc) return rc;
     if (strip_mode) {
+        const bool strided = gemv_strided_ok(vec_kind, w->K, d.stage32 != 0);
+        const int waves = strided ? gemv_strided_waves(vec_kind) : kGemvWaves;
         const int part_off = (gemv_strip_part_off(w->K, d.stage32 != 0) + 15) / 16 * 16;
         const long long per_wg = (d.n_strips + n_wg - 1) / n_wg;
-        const int lds_strip = part_off + (int)per_wg * kGemvWaves * kStripCols * 4;
+        const int lds_strip = part_off + (int)per_wg * waves * kStripCols * 4;
         if (gemv_max_wg_per_cu(lds_strip) > 0) {
-            const hipError_t e = launch_gemv_strips_single(d, d.n_strips, n_wg, lds_strip, part_off,
+            const hipError_t e = launch_gemv_strips_single(d, d.n_strips, n_wg, lds_strip, part_off, vec_kind, strided,
                                                            static_cast<hipStream_t>(stream));
             if (e != hipSuccess) return hip_fail(e, "gemv launch");
             return TER_HIP_OK;
         }
     }
     const int lds = gemv_t16_lds_bytes(w->K, d.stage32 != 0);
-    rc = pick_wg(total, 0, lds, prologue, -1, &n_wg);
+    rc = pick_wg(total, 0, lds, prologue, vec_kind, &n_wg);
     if (rc) return rc;
-    hipError_t e = launch_gemv(d, nullptr, nullptr, nullptr, total, n_wg, lds, -1, static_cast<hipStream_t>(stream));
+    hipError_t e =
+        launch_gemv(d, nullptr, nullptr, nullptr, total, n_wg, lds, vec_kind, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "gemv launch");
     return TER_HIP_OK;
 }
@@ -1392,31 +1453,7 @@ static int gemm_out_ws(const ter_hip_wpk_t* w, const ter_hip_act_t* x, int32_t M
         xq = q_ws;
         xs = s_ws;
     }
-    const bool vec = ring_rows_ok(xq, w->K);
-    int cus = 0;
-    rc = current_cu_count(&cus);
-    if (rc) return rc;
-    const GemmDesc whole = make_gemm_desc(w, xq, xs, M, *out);
-    const GemmPick pick = pick_gemm(&whole, 1, M, vec, cus);
-    if (pick.ring) {
-        const int mb = gemm_mb_of(std::min(M, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
-        // pieces of kRingRows rows, one LDS-ring launch each
-        for (int r0 = 0; r0 < M; r0 += kRingRows) {
-            const int m = std::min(kRingRows, M - r0);
-            const GemmDesc d = make_gemm_desc(w, xq + (size_t)r0 * w->K, xs + r0, m, out_rows(*out, r0, w->N));
-            const int nb = (d.n_strips + lbs - 1) / lbs;
-            int n_wg = 0;
-            rc = pick_lds_wg(nb, mb, &n_wg);
-            if (rc) return rc;
-            const hipError_t e = launch_gemm_lds(d, nullptr, nullptr, nullptr, nb, n_wg, mb, st);
-            if (e != hipSuccess) return hip_fail(e, "gemm launch");
-        }
-        return TER_HIP_OK;
-    }
-    const hipError_t e = launch_gemm_split(whole, nullptr, nullptr, 0, pick.tile, pick.longk, vec,
-                                           (long long)M * w->K < kSplitMinBytes, st);
-    if (e != hipSuccess) return hip_fail(e, "gemm launch");
-    return TER_HIP_OK;
+    return run_gemm(make_gemm_desc(w, xq, xs, M, *out), *out, st);
 }
 
 int ter_hip_gemm_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, int32_t M, const ter_hip_out_t* out,

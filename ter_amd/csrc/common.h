@@ -70,7 +70,8 @@ struct alignas(16) GemvDesc {
 struct alignas(16) GemmDesc {
     const uint8_t* w;            // T16 tile stream
     const int8_t* x;             // int8 [M][ldx]
-    const float* xs;             // per-row activation scales [M] (device)
+    const float* xs;             // per-row activation scales [M] (device), or null: x_scale (split kernel only)
+    float x_scale;
     float* y;                    // fp32 [M][N] or null
     int32_t* acc;                // int32 [M][N] or null
     uint16_t* y16;               // fp16 [M][N] = half(y) or null
@@ -102,9 +103,9 @@ bool gemv_strided_ok(int vec_kind, int32_t K, bool stage32);
 // Waves per workgroup of that prologue's kernel (its strips' partial sums
 // take [strip][waves][16] ints of LDS).
 int gemv_strided_waves(int vec_kind);
-// The same for one GEMV whose descriptor is a kernel argument (any activation kind).
+// The same for one GEMV whose descriptor is a kernel argument.
 hipError_t launch_gemv_strips_single(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
-                                     hipStream_t st);
+                                     int vec_kind, bool strided, hipStream_t st);
 // vec_kind: the activation kind of every GEMV of a work list that qualifies
 // for the vector prologue (gemv_vec_kind), else -1.
 // ranges_dev: [n_wg + 1] tile ranges of the workgroups of a work list (range

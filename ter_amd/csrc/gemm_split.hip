@@ -123,7 +123,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
         const int r0 = p * R;
         d.M -= r0;
         d.x += (long long)r0 * d.ldx;
-        d.xs += r0;
+        if (d.xs) d.xs += r0;
         const long long o = (long long)r0 * d.N;
         if (d.y) d.y += o;
         if (d.acc) d.acc += o;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
     constexpr int Q = R * 4 * C::BS, NQ = (Q + C::THREADS - 1) / C::THREADS;
     float xs[NQ];
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) xs[i] = gptr(d.xs)[min((tid + i * C::THREADS) / (4 * C::BS), M - 1)];
+    for (int i = 0; i < NQ; ++i) xs[i] = d.xs ? gptr(d.xs)[min((tid + i * C::THREADS) / (4 * C::BS), M - 1)] : d.x_scale;
 
     if (n > 0) stage(0, 0);
     load_x(0, D);

@@ -1703,41 +1703,50 @@ int gemv_max_wg_per_cu(int lds_bytes, int vec_kind) {
     return max_blocks_per_cu(fn, kGemvThreads, lds_bytes);
 }
 
+namespace {
+
+template <bool kList, int kKind>
+hipError_t launch_gemv_as(const GemvDesc& single, const GemvDesc* list_dev, const int32_t* first_dev,
+                          const long long* ranges_dev, long long total_tiles, int n_wg, int lds_bytes, hipStream_t st) {
+    hipLaunchKernelGGL((gemv_t16_kernel<kList, kKind>), dim3(n_wg), dim3(kGemvThreads), lds_bytes, st, single, list_dev,
+                       first_dev, ranges_dev, total_tiles, n_wg);
+    return hipGetLastError();
+}
+
+template <bool kList>
+hipError_t launch_gemv_kind(const GemvDesc& single, const GemvDesc* list_dev, const int32_t* first_dev,
+                            const long long* ranges_dev, long long total_tiles, int n_wg, int lds_bytes, int vec_kind,
+                            hipStream_t st) {
+    switch (vec_kind) {
+    case TER_HIP_X_I8:
+        return launch_gemv_as<kList, TER_HIP_X_I8>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg,
+                                                   lds_bytes, st);
+    case TER_HIP_X_F32:
+        return launch_gemv_as<kList, TER_HIP_X_F32>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg,
+                                                    lds_bytes, st);
+    case TER_HIP_X_F32_RMS:
+        return launch_gemv_as<kList, TER_HIP_X_F32_RMS>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg,
+                                                        lds_bytes, st);
+    case TER_HIP_X_F16_RMS:
+        return launch_gemv_as<kList, TER_HIP_X_F16_RMS>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg,
+                                                        lds_bytes, st);
+    case TER_HIP_X_RELU2_RMS:
+        return launch_gemv_as<kList, TER_HIP_X_RELU2_RMS>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg,
+                                                          lds_bytes, st);
+    default:
+        return launch_gemv_as<kList, -1>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg, lds_bytes, st);
+    }
+}
+
+}  // namespace
+
 hipError_t launch_gemv(const GemvDesc& single, const GemvDesc* list_dev, const int32_t* first_dev,
                        const long long* ranges_dev, long long total_tiles, int n_wg, int lds_bytes, int vec_kind,
                        hipStream_t st) {
-    const dim3 grid(n_wg), block(kGemvThreads);
-    if (!list_dev) {
-        hipLaunchKernelGGL((gemv_t16_kernel<false, -1>), grid, block, lds_bytes, st, single, list_dev, first_dev,
-                           ranges_dev, total_tiles, n_wg);
-        return hipGetLastError();
-    }
-    switch (vec_kind) {
-    case TER_HIP_X_I8:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, TER_HIP_X_I8>), grid, block, lds_bytes, st, single, list_dev,
-                           first_dev, ranges_dev, total_tiles, n_wg);
-        break;
-    case TER_HIP_X_F32:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, TER_HIP_X_F32>), grid, block, lds_bytes, st, single, list_dev,
-                           first_dev, ranges_dev, total_tiles, n_wg);
-        break;
-    case TER_HIP_X_F32_RMS:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, TER_HIP_X_F32_RMS>), grid, block, lds_bytes, st, single,
-                           list_dev, first_dev, ranges_dev, total_tiles, n_wg);
-        break;
-    case TER_HIP_X_F16_RMS:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, TER_HIP_X_F16_RMS>), grid, block, lds_bytes, st, single,
-                           list_dev, first_dev, ranges_dev, total_tiles, n_wg);
-        break;
-    case TER_HIP_X_RELU2_RMS:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, TER_HIP_X_RELU2_RMS>), grid, block, lds_bytes, st, single,
-                           list_dev, first_dev, ranges_dev, total_tiles, n_wg);
-        break;
-    default:
-        hipLaunchKernelGGL((gemv_t16_kernel<true, -1>), grid, block, lds_bytes, st, single, list_dev, first_dev,
-                           ranges_dev, total_tiles, n_wg);
-    }
-    return hipGetLastError();
+    return list_dev ? launch_gemv_kind<true>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg, lds_bytes,
+                                             vec_kind, st)
+                    : launch_gemv_kind<false>(single, list_dev, first_dev, ranges_dev, total_tiles, n_wg, lds_bytes,
+                                              vec_kind, st);
 }
 
 hipError_t launch_gemv_strips(const GemvDesc* list_dev, const GemvDesc* wg_desc_dev, long long total_strips, int n_wg,
@@ -1866,11 +1875,41 @@ bool gemv_strided_ok(int vec_kind, int32_t K, bool stage32) {
     }
 }
 
-hipError_t launch_gemv_strips_single(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
-                                     hipStream_t st) {
-    hipLaunchKernelGGL((gemv_strip_kernel<false, -1>), dim3(n_wg), dim3(kGemvThreads), lds_bytes, st, d, nullptr,
-                       nullptr, total_strips, n_wg, part_off);
+namespace {
+
+template <int kKind, bool kStrided>
+hipError_t launch_strip_single_as(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
+                                  hipStream_t st) {
+    constexpr int kW = kStrided ? strided_waves<kKind>() : kGemvWaves;
+    hipLaunchKernelGGL((gemv_strip_kernel<false, kKind, kStrided, kW>), dim3(n_wg), dim3(64 * kW), lds_bytes, st, d,
+                       nullptr, nullptr, total_strips, n_wg, part_off);
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemv_strips_single(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
+                                     int vec_kind, bool strided, hipStream_t st) {
+#define TER_SINGLE(kind, strided) launch_strip_single_as<kind, strided>(d, total_strips, n_wg, lds_bytes, part_off, st)
+    if (strided) {
+        switch (vec_kind) {
+        case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS, true);
+        case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS, true);
+        case TER_HIP_X_RELU2_RMS: return TER_SINGLE(TER_HIP_X_RELU2_RMS, true);
+        case TER_HIP_X_F16: return TER_SINGLE(TER_HIP_X_F16, true);
+        case TER_HIP_X_SILU_MUL: return TER_SINGLE(TER_HIP_X_SILU_MUL, true);
+        case TER_HIP_X_SMUL: return TER_SINGLE(TER_HIP_X_SMUL, true);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    switch (vec_kind) {
+    case TER_HIP_X_F32: return TER_SINGLE(TER_HIP_X_F32, false);
+    case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS, false);
+    case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS, false);
+    case TER_HIP_X_RELU2_RMS: return TER_SINGLE(TER_HIP_X_RELU2_RMS, false);
+    default: return TER_SINGLE(-1, false);
+    }
+#undef TER_SINGLE
 }
 
 }  // namespace terhip

@@ -475,6 +475,7 @@ struct ter_hip_plan {
     bool strip_mode = false;     // GEMV: strip-mode kernel, total counts strips
     int part_off = 0;            // GEMV strip mode: LDS offset of the partial sums
     bool strided = false;        // GEMV strip mode: the strided RMS prologue (gemv_strided_ok for every item)
+    int max_ku = 0;              //   and the largest Ku of its items
     bool shared = false;         // GEMV strided strip mode: one activation, back-to-back tile streams
     GemvDesc shared_desc{};      //   its kernel argument (shared_plan_desc)
     int mb = 0;                  // GEMM row-block count (LDS-ring kernel)
@@ -1312,6 +1313,7 @@ int ter_hip_plan_create(ter_hip_plan_t** plan, const ter_hip_gemv_item_t* items,
     p->strip_mode = strip_mode;
     p->part_off = part_off;
     p->strided = strip_mode && strided;
+    for (const GemvDesc& d : ds) p->max_ku = std::max(p->max_ku, (int)d.Ku);
     p->shared = shared;
     p->shared_desc = shared_desc;
     p->n_wg = n_wg;
@@ -1339,7 +1341,8 @@ int ter_hip_plan_launch(const ter_hip_plan_t* plan, void* stream) {
         if (plan->strip_mode)
             e = launch_gemv_strips(static_cast<const GemvDesc*>(plan->descs_dev),
                                    static_cast<const GemvDesc*>(plan->wg_desc_dev), plan->total,
-                                   plan->n_wg, plan->lds_bytes, plan->part_off, plan->vec_kind, plan->strided,
+                                   plan->n_wg, plan->lds_bytes, plan->part_off, plan->vec_kind,
+                                   plan->strided ? plan->max_ku : 0,
                                    plan->shared ? &plan->shared_desc : nullptr, static_cast<hipStream_t>(stream));
         else
             e = launch_gemv(none, static_cast<const GemvDesc*>(plan->descs_dev), plan->first_dev,

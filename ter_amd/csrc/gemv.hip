@@ -789,14 +789,15 @@ constexpr int strided_waves() {
 // The absmax kinds X_F16, X_SILU_MUL and X_SMUL (no sum, so no order to
 // keep): x (and up) of values 8 t + 8 T j, 8 halves per dwordx4 (X_SMUL: 8
 // fp32 x values in two).
-template <int kKind, int kW>
+template <int kKind, int kW, int kU>
 struct XStrided {
     static constexpr int T = 64 * kW;
     static constexpr bool R2 = kKind == TER_HIP_X_RELU2_RMS;
     static constexpr bool ABS = kKind == TER_HIP_X_F16 || kKind == TER_HIP_X_SILU_MUL || kKind == TER_HIP_X_SMUL;
     static constexpr bool UP = R2 || kKind == TER_HIP_X_SILU_MUL || kKind == TER_HIP_X_SMUL;
     static constexpr int V = R2 ? 1024 / T : (ABS ? 8 : 1);                                  // values per load
-    static constexpr int J = max_strided_ku<kKind>() * kUnitK / (R2 ? 1024 : (ABS ? 8 * T : T));  // loads per operand
+    static constexpr int J = kU * kUnitK / (R2 ? 1024 : (ABS ? 8 * T : T));  // loads per operand
+    static_assert(kU * kUnitK % (R2 ? 1024 : (ABS ? 8 * T : T)) == 0, "whole loads");
     static constexpr int DW = R2 ? (V + 1) / 2 : (ABS ? 4 : 1);                               // dwords per load
     static constexpr int DX = kKind == TER_HIP_X_SMUL ? 8 : DW;                              // dwords of x per load
     unsigned x[J][DX];  // fp32 bits (X_F32_RMS, X_SMUL) or fp16 bits (X_F16_RMS, X_F16; the gate of X_RELU2_RMS / X_SILU_MUL)
@@ -822,9 +823,9 @@ __device__ __forceinline__ void load_halves(__amdgpu_buffer_rsrc_t r, int off, u
     }
 }
 
-template <int kKind, int kW>
-__device__ __forceinline__ void x_prefetch_strided(const GemvDesc& d, XStrided<kKind, kW>& r) {
-    using XS = XStrided<kKind, kW>;
+template <int kKind, int kW, int kU>
+__device__ __forceinline__ void x_prefetch_strided(const GemvDesc& d, XStrided<kKind, kW, kU>& r) {
+    using XS = XStrided<kKind, kW, kU>;
     constexpr int J = XS::J, T = XS::T;
     const int t = threadIdx.x;
     const __amdgpu_buffer_rsrc_t rx = vec_rsrc(d.x, d.K * kind_bytes(kKind));
@@ -891,12 +892,12 @@ __device__ __forceinline__ void x_prefetch_strided(const GemvDesc& d, XStrided<k
 // a wave-level fence orders them before the loop.  Results are stage_x_vec's
 // bit for bit.  Needs Ku <= max_strided_ku and the fp32 staging (stage32);
 // gs16: fp16 gamma [Ku*256], red: 1024 + 16 floats.
-template <int kKind, int kW>
-__device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrided<kKind, kW>& r, int8_t* lds_x,
+template <int kKind, int kW, int kU>
+__device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrided<kKind, kW, kU>& r, int8_t* lds_x,
                                                  int* usum, float* red, float* xs32, uint16_t* gs16, int u0, int u1,
                                                  bool owner) {
 #pragma clang fp contract(off)
-    using XS = XStrided<kKind, kW>;
+    using XS = XStrided<kKind, kW, kU>;
     constexpr int J = XS::J, T = XS::T, V = XS::V;
     static_assert(XS::R2 ? (T == 256 || T == 512) : T == 256, "thread count");
     const int K = d.K, Ku = d.Ku;
@@ -905,6 +906,13 @@ __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrid
     float P[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) P[e] = 0.f;
+    // Values past the staged range are written too, x to the thread's own slots
+    // of `red`, which its partials overwrite below, gamma to the start of
+    // lds_x, which is written after the barriers: a branch per value cuts the
+    // loop into blocks, each of which waits for every load in flight, the
+    // first weight batch included.
+    float* const spare = red + (XS::R2 ? V * t : t);
+    uint16_t* const spare16 = reinterpret_cast<uint16_t*>(lds_x) + lane;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
 #pragma unroll
@@ -922,10 +930,9 @@ __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrid
             }
             P[e] = __builtin_fmaf(x[j][e], x[j][e], P[e]);  // past K: fma(0, 0, p) = p
             const int i = XS::R2 ? V * t + e + 1024 * j : t + T * j;
-            if (i < Ku * kUnitK) {  // the staged range
-                xs32[i] = x[j][e];
-                gs16[i] = XS::R2 ? gh : (uint16_t)r.g[j][0];
-            }
+            const bool in = i < Ku * kUnitK;  // the staged range
+            *(in ? xs32 + i : spare + e) = x[j][e];
+            *(in ? gs16 + i : spare16) = XS::R2 ? gh : (uint16_t)r.g[j][0];
         }
     }
 #pragma unroll
@@ -994,15 +1001,16 @@ __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrid
 // publishes xs32); each wave quantizes only its own units [u0, u1), as in
 // stage_x_strided.  The maximum is order-free, so the results are stage_x's
 // bit for bit.  Needs Ku <= max_strided_ku and the fp32 staging; red: kW floats.
-template <int kKind, int kW>
-__device__ __forceinline__ float stage_x_abs_strided(const GemvDesc& d, const XStrided<kKind, kW>& r, int8_t* lds_x,
+template <int kKind, int kW, int kU>
+__device__ __forceinline__ float stage_x_abs_strided(const GemvDesc& d, const XStrided<kKind, kW, kU>& r, int8_t* lds_x,
                                                      int* usum, float* red, float* xs32, int u0, int u1, bool owner) {
 #pragma clang fp contract(off)
-    using XS = XStrided<kKind, kW>;
+    using XS = XStrided<kKind, kW, kU>;
     constexpr int J = XS::J, T = XS::T;
     const int K = d.K, Ku = d.Ku;
     const int t = threadIdx.x, lane = t & 63;
     float mx = 0.f;  // zeros past K
+    float* const spare = red + 16 + 8 * lane;  // behind the waves' maxima
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         float v[8];
@@ -1022,10 +1030,11 @@ __device__ __forceinline__ float stage_x_abs_strided(const GemvDesc& d, const XS
             mx = fmaxf(mx, fabsf(v[e]));
         }
         const int i = 8 * t + 8 * T * j;
-        if (i < Ku * kUnitK) {  // the staged range (a multiple of 8)
-            *reinterpret_cast<f32x4*>(xs32 + i) = f32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4*>(xs32 + i + 4) = f32x4{v[4], v[5], v[6], v[7]};
-        }
+        // (the staged range is a multiple of 8; past it a slot nothing reads,
+        // for stage_x_strided's reason)
+        float* const o = i < Ku * kUnitK ? xs32 + i : spare;
+        *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(o + 4) = f32x4{v[4], v[5], v[6], v[7]};
     }
     mx = wave_max(mx);
     if (lane == 0) red[t >> 6] = mx;
@@ -1504,7 +1513,8 @@ void gemv_t16_kernel(GemvDesc single,
 // strip's partial column sums in LDS, and after a barrier wave j % 4 adds the
 // four partials of strip j (integer sums, so the result is the stream-K
 // kernel's) and writes the outputs.  No fix-up slots, no global atomics.
-template <bool kList, int kKind, bool kStrided = false, int kW = kGemvWaves, bool kShared = false>
+// kU > 0: the strided prologue, for at most kU units of K.
+template <bool kList, int kKind, int kU = 0, int kW = kGemvWaves, bool kShared = false>
 __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, const GemvDesc* __restrict__ list,
                                                                   const GemvDesc* __restrict__ wg_desc,
                                                                   long long total, int n_wg, int part_off) {
@@ -1519,6 +1529,7 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
     // The range is one segment; it spans at most two GEMVs, whose
     // descriptors wg_desc holds per block index (2 b: the first, 2 b + 1:
     // the next), so their loads need no argument but the table's address.
+    constexpr bool kStrided = kU > 0;
     static_assert(!kShared || (kList && kStrided), "shared lists run the strided prologue");
     GemvDesc e0{}, e1{};
     if constexpr (kShared) {
@@ -1580,15 +1591,19 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
         };
         XPre xpre;
         XRaw xraw;
-        XStrided<kStrided ? kKind : TER_HIP_X_F32_RMS, kStrided ? kW : kGemvWaves> xst;
+        XStrided<kStrided ? kKind : TER_HIP_X_F32_RMS, kStrided ? kW : kGemvWaves, kStrided ? kU : 8> xst;
         if constexpr (kKind < 0)
             x_prefetch(d, xpre);
         else if constexpr (kStrided)
-            x_prefetch_strided<kKind, kW>(d, xst);
+            x_prefetch_strided<kKind, kW, kU>(d, xst);
         else
             x_prefetch_vec<kKind>(d, xraw);
         u32x4 wa[NB], wb[NB];
-        if (nw > 0) load_b(wa);
+        // (Also by a wave without units, which does not use them: where it is
+        // skipped the loads in flight are not known and the prologue waits for
+        // these too.  With the staging's stores likewise without branches, per
+        // Llama token 459 -> 424 us.)
+        load_b(wa);
         if constexpr (kShared) {
             // the descriptors the outputs need, in flight with the activation
             // and weight loads (left alone the compiler issues them at the
@@ -1608,10 +1623,10 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
         } else if constexpr (kStrided) {
             uint16_t* gs16 = reinterpret_cast<uint16_t*>(lds_raw + gemv_lds_slots_offset(d.K, true));
             float* red_s = reinterpret_cast<float*>(lds_raw + gemv_strip_red_offset(d.K));
-            if constexpr (XStrided<kKind, kW>::ABS)
-                act = stage_x_abs_strided<kKind, kW>(d, xst, lds_x, usum, red_s, xs32, u0, u0 + nw, sg == d.strip0);
+            if constexpr (XStrided<kKind, kW, kU>::ABS)
+                act = stage_x_abs_strided<kKind, kW, kU>(d, xst, lds_x, usum, red_s, xs32, u0, u0 + nw, sg == d.strip0);
             else
-                act = stage_x_strided<kKind, kW>(d, xst, lds_x, usum, red_s, xs32, gs16, u0, u0 + nw,
+                act = stage_x_strided<kKind, kW, kU>(d, xst, lds_x, usum, red_s, xs32, gs16, u0, u0 + nw,
                                                  sg == d.strip0);
         } else {
             act = stage_x_vec<kKind>(d, xraw, lds_x, usum, red, xs32, sg == d.strip0);
@@ -1749,81 +1764,58 @@ hipError_t launch_gemv(const GemvDesc& single, const GemvDesc* list_dev, const i
                                               vec_kind, st);
 }
 
+namespace {
+
+// One strided strip launch: kMode 0 a single GEMV (`d`), 1 a list, 2 a shared list.
+template <int kMode, int kKind, int kU>
+hipError_t launch_strided_as(const GemvDesc& d, const GemvDesc* list_dev, const GemvDesc* wg_desc_dev,
+                             long long total_strips, int n_wg, int lds_bytes, int part_off, hipStream_t st) {
+    constexpr int kW = strided_waves<kKind>();
+    hipLaunchKernelGGL((gemv_strip_kernel<kMode != 0, kKind, kU, kW, kMode == 2>), dim3(n_wg), dim3(64 * kW), lds_bytes,
+                       st, d, list_dev, wg_desc_dev, total_strips, n_wg, part_off);
+    return hipGetLastError();
+}
+
+// The prologue's loads and arithmetic are unrolled for kU units of K, so the
+// smallest bound that holds the list's longest K is taken (the BitNet layer's
+// 10- and 27-unit lists: 39.3 us against bounds of 16 and 32, 38.9 with these;
+// the Llama token's 8- and 32-unit lists 458 us with either).
+template <int kMode>
+hipError_t launch_strided(const GemvDesc& d, const GemvDesc* list_dev, const GemvDesc* wg_desc_dev,
+                          long long total_strips, int n_wg, int lds_bytes, int part_off, int kind, int ku,
+                          hipStream_t st) {
+#define TER_STRIDED(kind, u) \
+    launch_strided_as<kMode, kind, u>(d, list_dev, wg_desc_dev, total_strips, n_wg, lds_bytes, part_off, st)
+    switch (kind) {
+    case TER_HIP_X_F32_RMS:
+        return ku <= 8 ? TER_STRIDED(TER_HIP_X_F32_RMS, 8)
+                       : (ku <= 10 ? TER_STRIDED(TER_HIP_X_F32_RMS, 10) : TER_STRIDED(TER_HIP_X_F32_RMS, 16));
+    case TER_HIP_X_F16_RMS:
+        return ku <= 8 ? TER_STRIDED(TER_HIP_X_F16_RMS, 8)
+                       : (ku <= 10 ? TER_STRIDED(TER_HIP_X_F16_RMS, 10) : TER_STRIDED(TER_HIP_X_F16_RMS, 16));
+    case TER_HIP_X_RELU2_RMS:
+        return ku <= 16 ? TER_STRIDED(TER_HIP_X_RELU2_RMS, 16)
+                        : (ku <= 28 ? TER_STRIDED(TER_HIP_X_RELU2_RMS, 28) : TER_STRIDED(TER_HIP_X_RELU2_RMS, 32));
+    case TER_HIP_X_F16: return ku <= 8 ? TER_STRIDED(TER_HIP_X_F16, 8) : TER_STRIDED(TER_HIP_X_F16, 16);
+    case TER_HIP_X_SILU_MUL:
+        return ku <= 16 ? TER_STRIDED(TER_HIP_X_SILU_MUL, 16) : TER_STRIDED(TER_HIP_X_SILU_MUL, 32);
+    case TER_HIP_X_SMUL: return ku <= 16 ? TER_STRIDED(TER_HIP_X_SMUL, 16) : TER_STRIDED(TER_HIP_X_SMUL, 32);
+    default: return hipErrorInvalidValue;
+    }
+#undef TER_STRIDED
+}
+
+}  // namespace
+
 hipError_t launch_gemv_strips(const GemvDesc* list_dev, const GemvDesc* wg_desc_dev, long long total_strips, int n_wg,
-                              int lds_bytes, int part_off, int vec_kind, bool strided, const GemvDesc* shared,
+                              int lds_bytes, int part_off, int vec_kind, int strided_ku, const GemvDesc* shared,
                               hipStream_t st) {
     const dim3 grid(n_wg), block(kGemvThreads);
-    if (strided && shared) {
-        switch (vec_kind) {
-        case TER_HIP_X_F32_RMS:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F32_RMS, true, kGemvWaves, true>), grid, block,
-                               lds_bytes, st, *shared, list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_F16_RMS:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F16_RMS, true, kGemvWaves, true>), grid, block,
-                               lds_bytes, st, *shared, list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_RELU2_RMS:
-            hipLaunchKernelGGL(
-                (gemv_strip_kernel<true, TER_HIP_X_RELU2_RMS, true, strided_waves<TER_HIP_X_RELU2_RMS>(), true>),
-                grid, dim3(64 * strided_waves<TER_HIP_X_RELU2_RMS>()), lds_bytes, st, *shared, list_dev, wg_desc_dev,
-                total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_F16:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F16, true, strided_waves<TER_HIP_X_F16>(), true>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_F16>()), lds_bytes, st, *shared, list_dev,
-                               wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_SILU_MUL:
-            hipLaunchKernelGGL(
-                (gemv_strip_kernel<true, TER_HIP_X_SILU_MUL, true, strided_waves<TER_HIP_X_SILU_MUL>(), true>),
-                grid, dim3(64 * strided_waves<TER_HIP_X_SILU_MUL>()), lds_bytes, st, *shared, list_dev, wg_desc_dev,
-                total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_SMUL:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_SMUL, true, strided_waves<TER_HIP_X_SMUL>(), true>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_SMUL>()), lds_bytes, st, *shared, list_dev,
-                               wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        default:
-            return hipErrorInvalidValue;
-        }
-    }
-    if (strided) {
-        const GemvDesc sh{};
-        switch (vec_kind) {
-        case TER_HIP_X_F32_RMS:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F32_RMS, true>), grid, block, lds_bytes, st,
-                               sh, list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_F16_RMS:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F16_RMS, true>), grid, block, lds_bytes, st,
-                               sh, list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_RELU2_RMS:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_RELU2_RMS, true, strided_waves<TER_HIP_X_RELU2_RMS>()>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_RELU2_RMS>()), lds_bytes, st, sh,
-                               list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_F16:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_F16, true, strided_waves<TER_HIP_X_F16>()>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_F16>()), lds_bytes, st, sh,
-                               list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_SILU_MUL:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_SILU_MUL, true, strided_waves<TER_HIP_X_SILU_MUL>()>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_SILU_MUL>()), lds_bytes, st, sh,
-                               list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        case TER_HIP_X_SMUL:
-            hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_SMUL, true, strided_waves<TER_HIP_X_SMUL>()>),
-                               grid, dim3(64 * strided_waves<TER_HIP_X_SMUL>()), lds_bytes, st, sh,
-                               list_dev, wg_desc_dev, total_strips, n_wg, part_off);
-            return hipGetLastError();
-        default:
-            return hipErrorInvalidValue;
-        }
-    }
+    if (strided_ku > 0)
+        return shared ? launch_strided<2>(*shared, list_dev, wg_desc_dev, total_strips, n_wg, lds_bytes, part_off,
+                                          vec_kind, strided_ku, st)
+                      : launch_strided<1>(GemvDesc{}, list_dev, wg_desc_dev, total_strips, n_wg, lds_bytes, part_off,
+                                          vec_kind, strided_ku, st);
     switch (vec_kind) {
     case TER_HIP_X_I8:
         hipLaunchKernelGGL((gemv_strip_kernel<true, TER_HIP_X_I8>), grid, block, lds_bytes, st, GemvDesc{},
@@ -1877,12 +1869,11 @@ bool gemv_strided_ok(int vec_kind, int32_t K, bool stage32) {
 
 namespace {
 
-template <int kKind, bool kStrided>
+template <int kKind>
 hipError_t launch_strip_single_as(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
                                   hipStream_t st) {
-    constexpr int kW = kStrided ? strided_waves<kKind>() : kGemvWaves;
-    hipLaunchKernelGGL((gemv_strip_kernel<false, kKind, kStrided, kW>), dim3(n_wg), dim3(64 * kW), lds_bytes, st, d,
-                       nullptr, nullptr, total_strips, n_wg, part_off);
+    hipLaunchKernelGGL((gemv_strip_kernel<false, kKind>), dim3(n_wg), dim3(kGemvThreads), lds_bytes, st, d, nullptr,
+                       nullptr, total_strips, n_wg, part_off);
     return hipGetLastError();
 }
 
@@ -1890,24 +1881,15 @@ hipError_t launch_strip_single_as(const GemvDesc& d, long long total_strips, int
 
 hipError_t launch_gemv_strips_single(const GemvDesc& d, long long total_strips, int n_wg, int lds_bytes, int part_off,
                                      int vec_kind, bool strided, hipStream_t st) {
-#define TER_SINGLE(kind, strided) launch_strip_single_as<kind, strided>(d, total_strips, n_wg, lds_bytes, part_off, st)
-    if (strided) {
-        switch (vec_kind) {
-        case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS, true);
-        case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS, true);
-        case TER_HIP_X_RELU2_RMS: return TER_SINGLE(TER_HIP_X_RELU2_RMS, true);
-        case TER_HIP_X_F16: return TER_SINGLE(TER_HIP_X_F16, true);
-        case TER_HIP_X_SILU_MUL: return TER_SINGLE(TER_HIP_X_SILU_MUL, true);
-        case TER_HIP_X_SMUL: return TER_SINGLE(TER_HIP_X_SMUL, true);
-        default: return hipErrorInvalidValue;
-        }
-    }
+    if (strided)
+        return launch_strided<0>(d, nullptr, nullptr, total_strips, n_wg, lds_bytes, part_off, vec_kind, d.Ku, st);
+#define TER_SINGLE(kind) launch_strip_single_as<kind>(d, total_strips, n_wg, lds_bytes, part_off, st)
     switch (vec_kind) {
-    case TER_HIP_X_F32: return TER_SINGLE(TER_HIP_X_F32, false);
-    case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS, false);
-    case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS, false);
-    case TER_HIP_X_RELU2_RMS: return TER_SINGLE(TER_HIP_X_RELU2_RMS, false);
-    default: return TER_SINGLE(-1, false);
+    case TER_HIP_X_F32: return TER_SINGLE(TER_HIP_X_F32);
+    case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS);
+    case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS);
+    case TER_HIP_X_RELU2_RMS: return TER_SINGLE(TER_HIP_X_RELU2_RMS);
+    default: return TER_SINGLE(-1);
     }
 #undef TER_SINGLE
 }

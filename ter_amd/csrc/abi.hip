@@ -1010,7 +1010,9 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
         // MFMA's sixteen rows are padding, but these launches are bound by
         // latency and HBM; in graphs: 2560 x 640 3.4 against 4.5 us, 6912 x 2560
         // 4.4 against 6.0, 2048 x 128256 13.4 against 16.1, unaligned 1003 x
-        // 1236 3.4 against 5.1).  With a host scale the ring kernel is out
+        // 1236 3.4 against 5.1; over weights that are not in the caches 2048 x
+        // 512 3.3 against 4.6, 6912 x 2560 5.7 against 5.9, 8192 x 2048 6.0
+        // against 5.9).  With a host scale the ring kernel is out
         // (it loads device scales), and past strip mode's size the stream-K
         // kernel takes over from the split one.
         GemmDesc gd = make_gemm_desc(w, static_cast<const int8_t*>(x->data), x->scale_dev, 1, *out);

@@ -688,14 +688,17 @@ __global__ void done_kernel(uint32_t* done, uint32_t call) {
 // Waits for the call's done_kernel by reading its number: a call takes 13.2 us
 // at K = 256, N = 64 (15.8 at 2560 x 6912), where it took 16.8 (19.4) with
 // hipStreamSynchronize and 20-25 polling hipStreamQuery.  After kDoneWait (a
-// stream with much other work in front, or a failed launch) the stream is
+// stream with much other work in front, or a kernel that failed) the stream is
 // synchronized instead, which also reports errors.
 constexpr std::chrono::microseconds kDoneWait(200);
 static hipError_t wait_done(MmRowStage& s, hipStream_t st) {
     const uint32_t call = ++s.calls;
     hipLaunchKernelGGL(done_kernel, dim3(1), dim3(1), 0, st, s.done_dev, call);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(st);  // the upload and the GEMV still use the staging
+        return e;
+    }
     const auto until = std::chrono::steady_clock::now() + kDoneWait;
     while (*s.done != call) {
         for (int i = 0; i < 64 && *s.done != call; ++i) __builtin_ia32_pause();
@@ -1113,7 +1116,10 @@ int ter_hip_mm_row(const int32_t* X, int32_t row, int32_t K, float x_scale, cons
         e = hipMemcpyAsync(x_stage_dev, sg->x, xbytes, hipMemcpyHostToDevice, st);
         if (e != hipSuccess) return hip_fail(e, "X upload");
         int rc = ter_hip_gemv(W, &x, sg->y_dev, nullptr, stream);
-        if (rc) return rc;
+        if (rc) {
+            (void)hipStreamSynchronize(st);  // the upload still reads the staging
+            return rc;
+        }
         e = wait_done(*sg, st);
         if (e != hipSuccess) return hip_fail(e, "mm_row synchronize");
         std::memcpy(out, sg->y, (size_t)N * sizeof(float));

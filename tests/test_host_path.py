@@ -1,0 +1,79 @@
+"""The library's host code on the CPU, over a HIP runtime that runs no kernels
+(tests/c/fake_hip.cpp): what a call launches, copies and waits for."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+fake.fake_log.restype = C.c_char_p
+fake.fake_fail.argtypes = [C.c_char_p]
+from ter_amd import _lib as L
+lib = C.CDLL(L.LIB_PATH)
+for name, res, args in L.SIGNATURES:
+    f = getattr(lib, name)
+    f.restype, f.argtypes = res, args
+keep = []
+def buf(n):
+    b = C.create_string_buffer(n + 4096)
+    keep.append(b)
+    return (C.addressof(b) + 4095) // 4096 * 4096
+def log():
+    lines = fake.fake_log().decode().splitlines()
+    fake.fake_reset()
+    return lines
+def weight(K, N):
+    w = L.WPK()
+    nb = lib.ter_hip_wpk_bytes(K, N)
+    assert lib.ter_hip_wpk_init(C.byref(w), buf(nb), nb, K, N, 0.5) == 0, lib.ter_hip_last_error()
+    keep.append(w)
+    return w
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    """The fake runtime, built; returns a function that runs a body over it in a fresh process."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not installed")
+    so = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    src = os.path.join(ROOT, "tests", "c", "fake_hip.cpp")
+    subprocess.run([gxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", src, "-o", so], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), so], cwd=ROOT, text=True,
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, timeout=120)
+        assert r.returncode == 0, r.stdout
+        return r.stdout
+
+    return run
+
+
+@pytest.mark.parametrize("xmax", [100, 9000], ids=["int8", "int16"])
+@pytest.mark.parametrize("kernel", ["done_kernel", "gem"], ids=["number", "product"])
+def test_mm_row_waits_before_a_launch_error(fake, kernel, xmax):
+    """A launch that fails leaves the row's upload (and the product) in flight
+    on the buffers that the next call takes over: the call waits for the
+    stream before it gives them up."""
+    fake(f"""
+    K, N = 512, 64
+    W = weight(K, N)
+    X = (C.c_int32 * K)(*[{xmax}] * K)
+    out, xs, ys = (C.c_float * N)(), buf(2 * K), buf(4 * N)
+    call = lambda: lib.ter_hip_mm_row(C.addressof(X), 0, K, 0.01, C.byref(W), N, C.addressof(out), xs, ys, None)
+    assert call() == 0
+    ran = log()
+    assert "done_kernel" in ran[-1] and not any(l.startswith("sync") for l in ran), ran
+    fake.fake_fail(b"{kernel}")
+    assert call() == L.ERR_HIP
+    ran = log()
+    assert ran[-2].startswith("failed") and ran[-1].startswith("sync"), ran
+    """)

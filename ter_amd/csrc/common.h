@@ -19,6 +19,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <atomic>
+#include <initializer_list>
 #include <type_traits>
 #include <stdint.h>
 
@@ -480,6 +482,27 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int hip_fail(hipError_t e, const char* what);
 
 int device_cu_count(int device);
+// Raises the limit on a launch's dynamic LDS (64 KiB by default) for some
+// kernels, once for each device that they run on; failures are not kept.
+class LdsLimit {
+public:
+    hipError_t allow(int bytes, std::initializer_list<const void*> kernels) {
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const uint64_t bit = dev < 64 ? 1ull << dev : 0ull;
+        if (done_.load(std::memory_order_acquire) & bit) return hipSuccess;
+        for (const void* k : kernels) {
+            e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+            if (e != hipSuccess) return e;
+        }
+        done_.fetch_or(bit, std::memory_order_release);
+        return hipSuccess;
+    }
+
+private:
+    std::atomic<uint64_t> done_{0};
+};
 // Resident workgroups per CU of a kernel at this LDS size (0 if the query fails).
 int max_blocks_per_cu(const void* fn, int threads, int lds_bytes);
 // Resident GEMV workgroups per CU at this LDS size (0 if the query fails).

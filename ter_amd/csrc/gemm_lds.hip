@@ -768,19 +768,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_lds_kernel(GemmDesc single, c
     }
 }
 
-// Allow the configuration's dynamic LDS (above the 64 KiB default) for both
-// instantiations; once per process (repeating it is harmless).
+// Allow the configuration's dynamic LDS for both instantiations.
 template <class C>
 hipError_t allow_lds() {
-    static hipError_t done = [] {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_lds_kernel<C, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_lds_kernel<C, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-        return e;
-    }();
-    return done;
+    static LdsLimit limit;
+    return limit.allow(C::LDS, {reinterpret_cast<const void*>(&gemm_lds_kernel<C, true>),
+                                reinterpret_cast<const void*>(&gemm_lds_kernel<C, false>)});
 }
 
 template <class C>

@@ -321,11 +321,9 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
 template <class C, int kX, bool kList>
 hipError_t launch_as(const GemmDesc& single, const GemmDesc* list, const GemmBlock* blocks, int n_blocks,
                      hipStream_t st) {
-    // dynamic LDS above the 64 KiB default, once per instantiation
-    static const hipError_t allowed =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_split_kernel<C, kX, kList>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-    if (allowed != hipSuccess) return allowed;
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(C::LDS, {reinterpret_cast<const void*>(&gemm_split_kernel<C, kX, kList>)});
+    if (e != hipSuccess) return e;
     const int n_sb = (single.n_strips + C::BS - 1) / C::BS, pieces = (single.M + C::R - 1) / C::R;
     const int grid = kList ? n_blocks : 8 * ((n_sb + 7) / 8) * pieces;
     hipLaunchKernelGGL((gemm_split_kernel<C, kX, kList>), dim3(grid), dim3(C::THREADS), C::LDS, st, single, list,

@@ -362,16 +362,10 @@ hipError_t launch_quant_as(const void* x, const uint16_t* up, const uint16_t* ga
     const int lds = KIND == TER_HIP_X_F32 ? 0 : (8 * T * NC + (KIND == TER_HIP_X_RELU2_RMS ? 1024 : 256)) * 4;
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     const bool vec = K % 8 == 0 && a16(x) && a16(up) && a16(gamma) && (reinterpret_cast<uintptr_t>(q) & 7u) == 0;
-    // dynamic LDS above the 64 KiB default, once per instantiation
-    static const hipError_t allowed = [lds] {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, false>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        return e;
-    }();
-    if (allowed != hipSuccess) return allowed;
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(lds, {reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, true>),
+                                           reinterpret_cast<const void*>(&quant_rows_kernel<T, NC, KIND, false>)});
+    if (e != hipSuccess) return e;
     if (vec)
         hipLaunchKernelGGL((quant_rows_kernel<T, NC, KIND, true>), dim3(M), dim3(T), lds, st, x, up, gamma, eps, K, q, s);
     else

@@ -77,3 +77,31 @@ def test_mm_row_waits_before_a_launch_error(fake, kernel, xmax):
     ran = log()
     assert ran[-2].startswith("failed") and ran[-1].startswith("sync"), ran
     """)
+
+
+@pytest.mark.parametrize("call,kernel", [
+    ("lib.ter_hip_rmsnorm_quant(x, L.X_F32_RMS, x, 1e-5, 8, 16384, q, s, None)", "quant_rows_kernel"),
+    ("lib.ter_hip_gemm(C.byref(W), C.byref(a), 256, y, None, None)", "gemm_split_kernel"),
+    ("lib.ter_hip_gemm(C.byref(WL), C.byref(a), 64, y, None, None)", "gemm_lds_kernel"),
+], ids=["rms_rows", "split", "ring"])
+def test_large_lds_is_allowed_on_each_device(fake, call, kernel):
+    """Kernels of more than 64 KiB of LDS: the limit is raised on the device of
+    the call, once for each, and before the first launch there."""
+    fake(f"""
+    W, WL = weight(256, 6912), weight(256, 65536)
+    x, q, s = buf(8 * 16384 * 4), buf(8 * 16384), buf(4096)
+    a = L.Act()
+    a.data, a.kind, a.scale_dev = buf(256 * 256), L.X_I8, s
+    y = buf(64)
+    for dev in (0, 1, 0, 1):
+        fake.fake_device(dev)
+        assert {call} == 0, lib.ter_hip_last_error()
+    ran = log()
+    launches = [l.split(" ", 5) for l in ran if l.startswith("launch") and "{kernel}" in l]
+    assert [l[1] for l in launches] == ["0", "1", "0", "1"], ran
+    for dev in "01":
+        _, _, _, _, lds, fn = launches[int(dev)]
+        at = [i for i, l in enumerate(ran) if l == f"attribute {{dev}} {{lds}} {{fn}}"]
+        assert int(lds) > 65536 and len(at) == 1, ran
+        assert at[0] < ran.index("launch " + " ".join(launches[int(dev)][1:])), ran
+    """)

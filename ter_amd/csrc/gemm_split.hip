@@ -211,6 +211,14 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
             *reinterpret_cast<u32x4*>(xd + (q * C::SG + sg) * 1024 + lane * 16) = a;
         }
     };
+    // the hand-over of a staged step between lanes (of one wave: no wait, the
+    // order alone)
+    auto stage_fence = [] {
+        if constexpr (C::SG > 1)
+            lds_barrier();
+        else
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
     i32x4 acc[S][MBW];
 #pragma unroll
     for (int s = 0; s < S; ++s)
@@ -234,7 +242,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
         for (int k = 0; k < D; ++k) {
             const int i = i0 + k;
             if (i < n_all) {
-                if constexpr (C::SG > 1) lds_barrier();
+                stage_fence();
                 const unsigned char* xd = xl + (C::NB > 1 ? (i & 1) * C::XB : 0);
                 i32x4 A[2][MBW];
 #pragma unroll
@@ -243,6 +251,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_split_kernel(GemmDesc single,
                     for (int mb = 0; mb < MBW; ++mb)
                         A[h][mb] = *reinterpret_cast<const i32x4*>(xd + (16 * mb + j) * kStepK +
                                                                    (((4 * h + g) ^ ((j >> 1) & 7)) * 16));
+                if constexpr (C::NB == 1) stage_fence();
                 if (i + 1 < n) stage((k + 1) % D, i + 1);
                 __builtin_amdgcn_sched_barrier(0);
                 if (i < n) {

@@ -241,25 +241,54 @@ int act_vec_kind(const ter_hip_act_t& x, int K) {
     return x.kind;
 }
 
+// Strip mode for work lists below kSmallPlanTilesPerWg tiles per workgroup at
+// the default occupancy and with at most four strips per CU (the decode
+// step's gate/up list, 2 x 432 strips of 10 units, included: 1.168 -> 1.147 ms
+// per C5 token against its stream-K partition).
+bool strip_mode_ok(long long total_tiles, long long total_strips, int cus) {
+    return total_tiles < (long long)cus * kGemvWgPerCu * kSmallPlanTilesPerWg && total_strips <= (long long)cus * 4;
+}
+
+// Whether a single GEMV on int8 rows runs the GEMM kernels at M = 1 (which
+// need no prologue; fifteen of an MFMA's sixteen rows are padding) instead of
+// the GEMV kernels with the int8 prologue.  In graphs, GEMM against GEMV, over
+// weights from HBM (over cached ones):
+//   vec rows, strip mode: 256 x 640 3.3 against 3.7 us (2.6, 2.9), 1024 x 4096
+//     3.75, 3.83 (2.8, 3.05), but 1024 x 8192 4.35, 4.23 (3.25, 3.4), 2560 x 640
+//     4.5, 4.0 (3.2, 3.2), 6912 x 2560 6.2, 4.9: GEMM for the shortest only.
+//   vec rows past strip mode (stream-K): at most two strips per CU 8192 x 8192
+//     8.4, 8.15 (6.3, 7.1), 12288 x 8192 9.9, 10.0 (7.3, 8.8), but 16384 x 8192
+//     12.1, 11.5; up to four strips per CU 6912 x 12288 11.0, 9.0; beyond (ring
+//     kernel and its device scales) 3072 x 24576 8.1, 8.9 and 4096 x 24576 11.4,
+//     9.8; 2048 x 32768 8.1, 8.1 and 2560 x 32768 9.5, 8.9; 2048 x 128256 14.1,
+//     16.6, 4096 x 128256 27.0, 27.3 and 8192 x 128256 50.9, 46.2.
+//   other rows (the general prologue): at most two strips per CU 3501 x 8192
+//     7.4, 8.0 (5.4, 7.2), but 4001 x 8192 7.6, 7.0; up to four 1003 x 16384
+//     6.6, 7.4, but 1501 x 16384 8.1, 7.7; more 255 x 32768 8.3, 7.3.
+bool int8_gemv_on_gemm(long long strips, int Ku, bool vec, bool dev_scale, int cus) {
+    const long long rounds = (strips + cus - 1) / cus;
+    if (!vec) return rounds <= 2 ? Ku <= 14 : rounds <= 4 && Ku <= 4;
+    if (strip_mode_ok(strips * Ku, strips, cus)) return Ku * rounds <= 4;
+    if (rounds <= 2) return Ku <= 48;
+    if (rounds <= 4 || !dev_scale) return false;
+    return Ku <= (strips >= 16LL * cus ? 16 : (strips >= 8LL * cus ? 8 : 12));
+}
+
 int gemv_vec_kind(const ter_hip_gemv_item_t* items, int n) {
     for (int i = 0; i < n; ++i)
         if (items[i].x.kind != items[0].x.kind || act_vec_kind(items[i].x, items[i].w->K) < 0) return -1;
     return items[0].x.kind;
 }
 
-// Strip mode for work lists below kSmallPlanTilesPerWg tiles per workgroup at
-// the default occupancy and with at most four strips per CU (the decode
-// step's gate/up list, 2 x 432 strips of 10 units, included: 1.168 -> 1.147 ms
-// per C5 token against its stream-K partition): one workgroup per strip up to
-// one per CU (two for int8 inputs, which have no prologue to repeat).
+// The workgroups of a launch in strip mode: one per strip up to one per CU (two
+// for int8 inputs, which have no prologue to repeat).
 int pick_strip_mode(long long total_tiles, long long total_strips, bool prologue, bool* strip_mode, int* n_wg) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
     const int cus = device_cu_count(dev);
     if (cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
-    *strip_mode = total_tiles < (long long)cus * kGemvWgPerCu * kSmallPlanTilesPerWg &&
-                  total_strips <= (long long)cus * 4;
+    *strip_mode = strip_mode_ok(total_tiles, total_strips, cus);
     if (!*strip_mode) return TER_HIP_OK;
     long long g = (long long)cus * (prologue ? 1 : kGemvWgPerCu);
     if (g > total_strips) g = total_strips;
@@ -1007,17 +1036,9 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
     int cus = 0;
     rc = current_cu_count(&cus);
     if (rc) return rc;
+    const int vec_kind = act_vec_kind(*x, w->K);
     if (x->kind == TER_HIP_X_I8 && !out->resid16 && !out->silu &&
-        (x->scale_dev || total < (long long)cus * kGemvWgPerCu * kSmallPlanTilesPerWg)) {
-        // int8 X needs no prologue: the GEMM kernels at M = 1 (fifteen of an
-        // MFMA's sixteen rows are padding, but these launches are bound by
-        // latency and HBM; in graphs: 2560 x 640 3.4 against 4.5 us, 6912 x 2560
-        // 4.4 against 6.0, 2048 x 128256 13.4 against 16.1, unaligned 1003 x
-        // 1236 3.4 against 5.1; over weights that are not in the caches 2048 x
-        // 512 3.3 against 4.6, 6912 x 2560 5.7 against 5.9, 8192 x 2048 6.0
-        // against 5.9).  With a host scale the ring kernel is out
-        // (it loads device scales), and past strip mode's size the stream-K
-        // kernel takes over from the split one.
+        int8_gemv_on_gemm(strips_of(w->N), units_of(w->K), vec_kind >= 0, x->scale_dev != nullptr, cus)) {
         GemmDesc gd = make_gemm_desc(w, static_cast<const int8_t*>(x->data), x->scale_dev, 1, *out);
         gd.x_scale = x->scale;
         return run_gemm(gd, *out, static_cast<hipStream_t>(stream));
@@ -1031,7 +1052,6 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
     // 5.6, fp16 absmax 5.9 -> 3.9 against the general one), and strip mode for
     // small GEMVs (whole strips per workgroup, the waves' partials added in
     // LDS, no fix-up slots)
-    const int vec_kind = act_vec_kind(*x, w->K);
     bool strip_mode = false;
     rc = pick_strip_mode(total, d.n_strips, prologue, &strip_mode, &n_wg);
     if (rc) return rc;

@@ -1896,6 +1896,7 @@ hipError_t launch_gemv_strips_single(const GemvDesc& d, long long total_strips, 
         return launch_strided<0>(d, nullptr, nullptr, total_strips, n_wg, lds_bytes, part_off, vec_kind, d.Ku, st);
 #define TER_SINGLE(kind) launch_strip_single_as<kind>(d, total_strips, n_wg, lds_bytes, part_off, st)
     switch (vec_kind) {
+    case TER_HIP_X_I8: return TER_SINGLE(TER_HIP_X_I8);
     case TER_HIP_X_F32: return TER_SINGLE(TER_HIP_X_F32);
     case TER_HIP_X_F32_RMS: return TER_SINGLE(TER_HIP_X_F32_RMS);
     case TER_HIP_X_F16_RMS: return TER_SINGLE(TER_HIP_X_F16_RMS);

@@ -87,3 +87,14 @@ def test_gemv_single_int8(cuda, K, N, shift, scale):
     one = np.float32(1)
     assert (r.cpu().numpy() == one + h.astype(np.float32)).all()
     assert (r16.cpu().numpy() == (one + h.astype(np.float32)).astype(np.float16)).all()
+
+
+# both sides of the lines between the GEMM kernels, strip mode and stream-K (256 CUs)
+ROUTES = [(1024, 4096), (1024, 4112), (1040, 64), (8192, 8176), (8192, 8192), (12288, 5472), (12304, 5472),
+          (1024, 16400), (3088, 16400), (2064, 32768), (3583, 8192), (3585, 64), (1025, 8208)]
+
+
+@pytest.mark.parametrize("scale", ["device", "host"])
+@pytest.mark.parametrize("K,N", ROUTES)
+def test_gemv_int8_routes(cuda, K, N, scale):
+    test_gemv_single_int8(cuda, K, N, 0, scale)

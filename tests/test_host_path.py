@@ -105,3 +105,34 @@ def test_large_lds_is_allowed_on_each_device(fake, call, kernel):
         assert int(lds) > 65536 and len(at) == 1, ran
         assert at[0] < ran.index("launch " + " ".join(launches[int(dev)][1:])), ran
     """)
+
+
+VEC_STRIP, STRIP = "gemv_strip_kernel<false, 0,", "gemv_strip_kernel<false, -1,"
+VEC_STREAM, STREAM, SPLIT, RING = "gemv_t16_kernel<false, 0>", "gemv_t16_kernel<false, -1>", "gemm_split", "gemm_lds"
+
+
+@pytest.mark.parametrize("K,N,shift,dev_scale,kernel", [
+    # 16-byte aligned rows, strip mode: the GEMM kernels for the shortest only
+    (1024, 4096, 0, 1, SPLIT), (1024, 4096, 0, 0, SPLIT), (1024, 4112, 0, 1, VEC_STRIP), (1040, 64, 0, 1, VEC_STRIP),
+    (2560, 640, 0, 1, VEC_STRIP), (2560, 640, 0, 0, VEC_STRIP), (32768, 2048, 0, 1, VEC_STREAM),
+    # past it: up to two strips per CU, up to four, eight, sixteen and more
+    (8192, 8176, 0, 1, VEC_STRIP), (8192, 8192, 0, 1, SPLIT), (12288, 5472, 0, 0, SPLIT), (12304, 5472, 0, 1, VEC_STREAM),
+    (4096, 16384, 0, 1, VEC_STREAM), (3072, 16400, 0, 0, VEC_STREAM), (3088, 16400, 0, 1, VEC_STREAM),
+    (2048, 32768, 0, 1, SPLIT), (2064, 32768, 0, 1, VEC_STREAM), (4096, 65536, 0, 1, RING), (4096, 65536, 0, 0, VEC_STREAM),
+    (4112, 65536, 0, 1, VEC_STREAM),
+    # other rows
+    (3583, 8192, 0, 1, SPLIT), (3585, 64, 0, 1, STRIP), (3584, 8192, 1, 0, SPLIT), (3600, 64, 1, 1, STRIP),
+    (1023, 16384, 0, 1, SPLIT), (1025, 8208, 0, 1, STRIP), (1023, 16400, 0, 1, STREAM), (15, 8, 0, 1, SPLIT),
+])
+def test_int8_gemv_route(fake, K, N, shift, dev_scale, kernel):
+    """Where a single int8 GEMV runs, on both sides of each line of its rule (256 CUs)."""
+    fake(f"""
+    W = weight({K}, {N})
+    a = L.Act()
+    a.data, a.kind, a.scale = buf({K} + 64) + {shift}, L.X_I8, 0.5
+    if {dev_scale}:
+        a.scale_dev = buf(4)
+    assert lib.ter_hip_gemv(C.byref(W), C.byref(a), buf({N} * 4), None, None) == 0, lib.ter_hip_last_error()
+    ran = [l for l in log() if l.startswith("launch")]
+    assert len(ran) == 1 and "{kernel}" in ran[0], ran
+    """)

@@ -379,11 +379,24 @@ double makespan(std::vector<double> costs, int slots) {
 // Split, one GEMM: its tiles take turns on the CUs (gemm_split_tile_us).  A
 // list: the longest tile, or the sum over the CUs times 1.4 (every CU reading
 // at once: at 8 layers and M = 128 the tiles cost 1.25-1.55 times their
-// single-GEMM time).  Ring: the list schedule's makespan, at a stage time
-// between that of few busy CUs and that of all (gemm_lds_unit_us).  Checked
-// for lists of 1-8 layers at M = 8-256 (BitNet-2B's shapes, and H = 768, F =
-// 2048 with up to 30 layers): the choice is the fastest of the seven, or
-// within 10% of it.
+// single-GEMM time).  Ring: the list schedule's makespan (one GEMM: a launch
+// per piece of rows), at a stage time between that of few busy CUs and that of
+// all (gemm_lds_unit_us).
+//
+// Both are fitted to weights in the caches.  A single GEMM of a model reads its
+// weights from HBM, where the split kernel, with two steps in flight per wave,
+// loses more than the ring; there, and with many rounds of 32 x 4 tiles, it has
+// to win by kSplitMargin.  Split against ring, weights from HBM (cached): M = 32,
+// 768 x 65536 11.7, 9.2 us (10.2, 9.0) and 2048 x 65536 15.8, 14.5 (13.0, 13.2); M
+// = 16, 4096 x 32768 12.2, 11.0 (9.9, 10.1); M = 128, 2048 x 32768 18.6, 17.3
+// (17.1, 17.4); M = 64, 2048 x 32768 10.9, 12.3 (9.6, 11.1).  Over 9 shapes at M =
+// 16-256 the choice is the faster one or within 9% of it.  The whole of a list
+// that is short enough for the split kernel stays in the Infinity Cache between
+// launches.  Over lists of 1-16 layers of four shapes at M = 2-256 the choice is
+// the faster one there or within 9% of it, and with weights from HBM at most 15%
+// from it (H = 1280, F = 5120, 4 layers, M = 2: 16.4 against 14.3 us, cached 12.8
+// against 13.0).
+constexpr double kSplitMargin = 1.3;
 struct GemmPick {
     bool ring;
     int tile;    // split kernel
@@ -423,14 +436,16 @@ GemmPick pick_gemm(const GemmDesc* whole, int n, int max_m, bool vec, int cus) {
         sum += (double)k * (whole[i].Ku + 1);
     }
     if (n == 1) {  // equal blocks
-        last = (double)((count + cus - 1) / cus) * (whole[0].Ku + 1);
+        const long long pieces = (whole[0].M + kRingRows - 1) / kRingRows, per = count / pieces;
+        last = (double)(pieces * ((per + cus - 1) / cus)) * (whole[0].Ku + 1);
     } else if (count > 8LL * cus) {  // a long list packs evenly
         last = sum / cus;
     } else {
         for (int i = 0; i < n; ++i) costs.insert(costs.end(), (size_t)blocks_of(i, kRingRows, lbs), whole[i].Ku + 1.0);
         last = makespan(costs, cus);
     }
-    best.ring = last * gemm_lds_unit_us(mb, std::min(1.0, sum / cus / last)) < best_us;
+    best.ring = last * gemm_lds_unit_us(mb, std::min(1.0, sum / cus / last)) <
+                (n == 1 ? kSplitMargin : 1.0) * best_us;
     return best;
 }
 

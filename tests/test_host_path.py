@@ -35,6 +35,26 @@ def weight(K, N):
     assert lib.ter_hip_wpk_init(C.byref(w), buf(nb), nb, K, N, 0.5) == 0, lib.ter_hip_last_error()
     keep.append(w)
     return w
+def gemm(M, K, N):  # the kernels one GEMM on int8 rows launches
+    a = L.Act()
+    a.data, a.kind, a.scale_dev = buf(M * K), L.X_I8, buf(4 * M)
+    W = weight(K, N)
+    log()
+    assert lib.ter_hip_gemm(C.byref(W), C.byref(a), M, buf(64), None, None) == 0, lib.ter_hip_last_error()
+    return [l for l in log() if l.startswith("launch")]
+def gemm_list(items, wg_per_cu=0):  # the kernel a list of GEMMs (M, K, N) launches, and the plan's workgroups
+    arr = (L.GemmItem * len(items))()
+    for it, (M, K, N) in zip(arr, items):
+        it.w, it.x, it.x_scale_dev, it.M, it.y = C.pointer(weight(K, N)), buf(M * K), buf(4 * M), M, buf(64)
+    p, n = C.c_void_p(), C.c_int32()
+    assert lib.ter_hip_gemm_plan_create(C.byref(p), arr, len(items), wg_per_cu) == 0, lib.ter_hip_last_error()
+    b, m = C.c_uint64(), C.c_uint64()
+    assert lib.ter_hip_plan_stats(p, C.byref(b), C.byref(m), C.byref(n)) == 0
+    log()
+    assert lib.ter_hip_plan_launch(p, None) == 0
+    ran = [l for l in log() if l.startswith("launch")]
+    assert len(ran) == 1, ran
+    return ran[0], n.value
 """
 
 
@@ -118,7 +138,7 @@ VEC_STREAM, STREAM, SPLIT, RING = "gemv_t16_kernel<false, 0>", "gemv_t16_kernel<
     # past it: up to two strips per CU, up to four, eight, sixteen and more
     (8192, 8176, 0, 1, VEC_STRIP), (8192, 8192, 0, 1, SPLIT), (12288, 5472, 0, 0, SPLIT), (12304, 5472, 0, 1, VEC_STREAM),
     (4096, 16384, 0, 1, VEC_STREAM), (3072, 16400, 0, 0, VEC_STREAM), (3088, 16400, 0, 1, VEC_STREAM),
-    (2048, 32768, 0, 1, SPLIT), (2064, 32768, 0, 1, VEC_STREAM), (4096, 65536, 0, 1, RING), (4096, 65536, 0, 0, VEC_STREAM),
+    (2048, 32768, 0, 1, RING), (2064, 32768, 0, 1, VEC_STREAM), (4096, 65536, 0, 1, RING), (4096, 65536, 0, 0, VEC_STREAM),
     (4112, 65536, 0, 1, VEC_STREAM),
     # other rows
     (3583, 8192, 0, 1, SPLIT), (3585, 64, 0, 1, STRIP), (3584, 8192, 1, 0, SPLIT), (3600, 64, 1, 1, STRIP),
@@ -135,4 +155,34 @@ def test_int8_gemv_route(fake, K, N, shift, dev_scale, kernel):
     assert lib.ter_hip_gemv(C.byref(W), C.byref(a), buf({N} * 4), None, None) == 0, lib.ter_hip_last_error()
     ran = [l for l in log() if l.startswith("launch")]
     assert len(ran) == 1 and "{kernel}" in ran[0], ran
+    """)
+
+
+def layers(n, M, H, F, q, kv):
+    return [(M, H, q), (M, H, kv), (M, H, kv), (M, q, H), (M, H, F), (M, H, F), (M, F, H)] * n
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (32, 768, 65536, RING), (16, 4096, 32768, RING), (128, 2048, 32768, RING), (64, 2048, 65536, RING),
+    (16, 2048, 16384, SPLIT), (64, 2560, 6912, SPLIT), (128, 8192, 8192, SPLIT), (256, 2560, 6912, SPLIT),
+    (256, 2048, 16384, SPLIT),
+])
+def test_gemm_route(fake, M, K, N, kernel):
+    """The kernel of a single GEMM (256 CUs): the faster one over weights from HBM."""
+    fake(f"""
+    ran = gemm({M}, {K}, {N})
+    assert ran and all("{kernel}" in l for l in ran), ran
+    """)
+
+
+@pytest.mark.parametrize("items,kernel", [
+    (layers(8, 128, 2560, 6912, 2560, 640), RING), (layers(4, 64, 2560, 6912, 2560, 640), RING),
+    (layers(3, 8, 2560, 6912, 2560, 640), RING), (layers(1, 32, 2560, 6912, 2560, 640), SPLIT),
+    (layers(4, 32, 2560, 6912, 2560, 640), SPLIT), (layers(2, 8, 2048, 8192, 2048, 512), SPLIT),
+], ids=["bitnet_x8_m128", "bitnet_x4_m64", "bitnet_x3_m8", "bitnet_x1_m32", "bitnet_x4_m32", "llama_x2_m8"])
+def test_gemm_list_route(fake, items, kernel):
+    """The same for lists."""
+    fake(f"""
+    ran, _ = gemm_list({items})
+    assert "{kernel}" in ran, ran
     """)

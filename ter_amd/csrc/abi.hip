@@ -407,7 +407,6 @@ GemmPick pick_gemm(const GemmDesc* whole, int n, int max_m, bool vec, int cus) {
     double best_us = 1e30;
     int max_ku = 0;
     for (int i = 0; i < n; ++i) max_ku = std::max(max_ku, whole[i].Ku);
-    best.longk = gemm_split_long(max_ku);
     auto blocks_of = [&](int i, int rows, int strips) {
         return (long long)((whole[i].M + rows - 1) / rows) * ((whole[i].n_strips + strips - 1) / strips);
     };
@@ -425,6 +424,7 @@ GemmPick pick_gemm(const GemmDesc* whole, int n, int max_m, bool vec, int cus) {
             best.tile = t;
         }
     }
+    best.longk = gemm_split_long(best.tile, max_ku, n == 1 && vec);
     if (!vec) return best;
     const int mb = gemm_mb_of(std::min(max_m, kRingRows)), lbs = gemm_lds_strips_per_block(mb);
     std::vector<double> costs;

@@ -207,7 +207,7 @@ int gemm_split_bytes_tile();
 int gemm_split_rows(int tile);
 int gemm_split_strips(int tile);
 float gemm_split_tile_us(int tile, int Ku);
-inline bool gemm_split_long(int Ku) { return Ku > 20; }
+bool gemm_split_long(int tile, int Ku, bool single_vec);  // single_vec: one GEMM, 16-byte aligned X rows
 hipError_t launch_gemm_split(const GemmDesc& single, const GemmDesc* list_dev, const GemmBlock* blocks_dev,
                              int n_blocks, int tile, bool longk, bool vec, bool bytes, hipStream_t st);
 

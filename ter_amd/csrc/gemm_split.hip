@@ -351,8 +351,7 @@ hipError_t launch_cfg(const GemmDesc& single, const GemmDesc* list, const GemmBl
 }
 
 // The tiles, largest first; the small ones also for long K (L: more K groups,
-// fewer steps per wave; K = 6912: 4.7 against 5.6 us at M = 16, 7.25 against
-// 7.8 at M = 64; K = 2560 the other way round, 3.6 against 3.4 us at M = 8).
+// fewer steps per wave; gemm_split_long).
 using T64x8 = SCfg<4, 1, 8, 2, 2>;
 using T64x4 = SCfg<4, 1, 4, 4, 2>;
 using T32x4 = SCfg<2, 1, 4, 4, 2>;
@@ -379,12 +378,22 @@ int gemm_split_strips(int tile) { return kTile[tile].strips; }
 
 // Time a tile over Ku 256-row units of K takes its CU beyond a launch's fixed
 // part, for the choice of the kernel and tile (pick_gemm in abi.hip): fitted
-// to HIP-event times of single GEMMs (3 us fixed; tiles beyond the CU count
-// take turns), which it gives within about 10% for M = 2-256, K = 256-8192, N
-// = 640-16384.  E.g. M = 64, 6912 x 2560: 7.6 (measured 7.25) as 32 x 2 tiles,
-// 9.7 (9.0) as 32 x 4; M = 256, 2560 x 6912: 10.2 (9.8) as 64 x 8, 12.1 (10.8)
-// as 64 x 4; M = 8, 2560 x 16384: 5.9 (5.1) as 16 x 2, 6.0 (5.9) as 16 x 1.
+// to HIP-event times of single GEMMs over cached weights (3 us fixed; tiles
+// beyond the CU count take turns), which it gives within about 16% for M =
+// 2-256, K = 256-8192, N = 640-16384.  E.g. M = 64, 6912 x 2560: 7.6 (measured
+// 7.25) as 32 x 2 tiles, 9.7 (9.0) as 32 x 4; M = 256, 2560 x 6912: 10.2 (9.8) as
+// 64 x 8, 12.1 (10.8) as 64 x 4; M = 8, 2560 x 16384: 5.9 (5.1) as 16 x 2, 6.0
+// (5.9) as 16 x 1.
 float gemm_split_tile_us(int tile, int Ku) { return kTile[tile].unit_us * (float)(Ku + 2); }
+
+// Whether a launch of this tile and largest Ku takes the long-K form.  Short
+// against long, weights from HBM (cached): one GEMM of 16 x 1 tiles at M = 8,
+// 2560 x 2560 4.9, 4.7 us (3.3, 3.4), 3328 x 4096 5.6, 5.1 (3.7, 3.6), 5120 x 4096
+// 6.7, 5.7 (4.1, 3.9); of 16 x 2 tiles 5120 x 8192 7.4, 7.0 (5.1, 5.2); of 32 x 2
+// at M = 64, 5120 x 2560 7.9, 8.6 (6.3, 6.4), 6144 x 2560 8.6, 8.7 (7.0, 6.6); rows
+// at any address, M = 16, 5001 x 2048 7.3, 7.8 (5.2, 5.8).  In a list the short
+// items pay for the long ones: K = 1024 and 4096, M = 8 6.9, 7.8 (5.0, 5.9).
+bool gemm_split_long(int tile, int Ku, bool single_vec) { return Ku > (single_vec && tile == kTiles - 1 ? 12 : 20); }
 
 hipError_t launch_gemm_split(const GemmDesc& single, const GemmDesc* list_dev, const GemmBlock* blocks_dev,
                              int n_blocks, int tile, bool longk, bool vec, bool bytes, hipStream_t st) {

@@ -186,3 +186,12 @@ def test_gemm_list_route(fake, items, kernel):
     ran, _ = gemm_list({items})
     assert "{kernel}" in ran, ran
     """)
+
+
+@pytest.mark.parametrize("M,K,N,groups", [(8, 3072, 640, 4), (8, 3088, 640, 8), (8, 5121, 640, 8), (8, 5119, 640, 4)])
+def test_gemm_split_long_k(fake, M, K, N, groups):
+    """The K groups of the 16 x 1 tile on both sides of its lines (aligned rows at 12 units of K, others at 20)."""
+    fake(f"""
+    ran = gemm({M}, {K}, {N})
+    assert len(ran) == 1 and "gemm_split" in ran[0] and "SCfg<1, 1, 1, {groups}, 2>" in ran[0], ran
+    """)

@@ -9,6 +9,7 @@ rounding of the exact integer times one rounded product of scales).
 import numpy as np
 import pytest
 
+from gemm_shapes import SPLIT_TAIL, SPLIT_TILES
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,20 @@ def test_gemm_split_ragged_columns(cuda):
     assert (acc.cpu().numpy() == ra).all()
     want = ra.astype(np.float32) * (xs * np.float32(0.02)).astype(np.float32)[:, None]
     assert (bits(y) == want.view(np.uint32)).all()
+
+
+# every tile with 16-byte loads, and at any address
+VEC = [(t, d) for t in SPLIT_TILES for d in (0, 1)]
+VEC_IDS = ["%dx%dx%d-%s" % (*t, "any" if d else "vec") for t, d in VEC]
+
+
+@pytest.mark.parametrize("tile,odd", VEC, ids=VEC_IDS)
+def test_gemm_split_tile_single(cuda, tile, odd):
+    M, K, N = SPLIT_TILES[tile][0]
+    test_gemm_split_single(cuda, M, K + odd, N, 0)
+
+
+@pytest.mark.parametrize("tile,odd", VEC, ids=VEC_IDS)
+def test_gemm_split_tile_list(cuda, tile, odd):
+    specs = [SPLIT_TILES[tile][1], SPLIT_TAIL]
+    test_gemm_split_list(cuda, [(M, K + odd, N) for M, K, N in specs], 0)

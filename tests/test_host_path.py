@@ -8,6 +8,8 @@ import textwrap
 
 import pytest
 
+from gemm_shapes import RING_LIST, RING_SINGLE, SPLIT_TAIL, SPLIT_TILES
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 PRELUDE = """
@@ -194,4 +196,34 @@ def test_gemm_split_long_k(fake, M, K, N, groups):
     fake(f"""
     ran = gemm({M}, {K}, {N})
     assert len(ran) == 1 and "gemm_split" in ran[0] and "SCfg<1, 1, 1, {groups}, 2>" in ran[0], ran
+    """)
+
+
+@pytest.mark.parametrize("odd", [0, 1], ids=["vec", "any"])
+def test_gemm_split_tiles_reached(fake, odd):
+    """The shapes of the GPU tests run every tile of the split kernel, in both load forms."""
+    fake(f"""
+    for (rows, strips, groups), (one, first) in {SPLIT_TILES}.items():
+        want = "gemm_split_kernel<terhip::(anonymous namespace)::SCfg<%d, 1, %d, %d, 2>, {2 - odd}, %s>"
+        M, K, N = one
+        ran = gemm(M, K + {odd}, N)
+        assert len(ran) == 1 and want % (rows // 16, strips, groups, "false") in ran[0], ran
+        ran, _ = gemm_list([(M, K + {odd}, N) for M, K, N in (first, {SPLIT_TAIL})])
+        assert want % (rows // 16, strips, groups, "true") in ran, ran
+        keep.clear()
+    """)
+
+
+def test_gemm_ring_reached(fake):
+    """Those of its tests run the ring kernel, with every count of row blocks."""
+    fake(f"""
+    import re
+    blocks = lambda l: int(re.search(r"gemm_lds_kernel<terhip::.anonymous namespace.::LCfg<(\\d+)", l)[1])
+    for M, K, N in {RING_SINGLE}:
+        ran = gemm(M, K, N)
+        assert len(ran) == -(-M // 128) and {{blocks(l) for l in ran}} == {{1 if M <= 16 else 2 if M <= 32 else 4 if M <= 64 else 8}}
+        keep.clear()
+    for name, items in {RING_LIST}.items():
+        assert blocks(gemm_list(items)[0]) == (8 if name == "pieces" else int(name))
+        keep.clear()
     """)

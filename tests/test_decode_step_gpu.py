@@ -181,10 +181,10 @@ def test_mm_packed_dispatch_f16(cuda):
 
 
 @pytest.mark.parametrize("M,aligned", [(8, True), (8, False), (32, True), (32, False), (100, True)],
-                         ids=["stream", "stream-bytewise", "lds-ring", "unit-major", "lds-ring-m100"])
+                         ids=["m8", "m8-unaligned", "m32", "m32-unaligned", "m100"])
 def test_gemm_f16_and_residual_outputs(cuda, M, aligned):
-    """Every GEMM kernel's epilogue: streaming (M <= 16), LDS ring (16-byte
-    rows), unit-major (X not 16-byte aligned)."""
+    """The split GEMM's fp16 and residual outputs at three row counts, X 16-byte
+    aligned and not (test_gemm_ring_gpu.py has the ring's)."""
     import torch
     import ter_amd as T
     K, N = 2560, 640

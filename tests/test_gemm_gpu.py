@@ -34,7 +34,7 @@ def assert_f32_equal(got, want):
 CASES = [
     (2, 300, 20), (8, 2560, 640), (16, 2048, 512), (17, 257, 36), (32, 2560, 640),
     (64, 640, 128), (128, 2560, 640), (200, 512, 48), (256, 256, 16), (8, 6912, 256),
-    (1, 2560, 640), (16, 6912, 64),  # M <= 16: streamed; M = 16 at K = 6912 exceeds its LDS and takes the row-block kernel
+    (1, 2560, 640), (16, 6912, 64),
 ]
 
 
@@ -78,11 +78,10 @@ def test_gemm_fp32_rows_quantized(cuda, M, K, N):
 
 
 def test_gemm_generated_shapes(cuda):
-    """Generated cases (hypothesis, derandomized): M from 2 to 256 (one to
-    two 128-row pieces, every row-block configuration), K from 1 to 3000
-    (16-byte aligned rows or not, so the LDS ring and the unaligned kernel
-    both run), N a multiple of 4 up to 600; single launches and a two-GEMM
-    plan; int32 and fp32 outputs against the oracle bit for bit."""
+    """Generated cases (hypothesis, derandomized): M from 2 to 256, K from 1 to
+    3000 (16-byte aligned rows or not, so the split kernel's load forms all
+    run), N a multiple of 4 up to 600; single launches and a two-GEMM plan;
+    int32 and fp32 outputs against the oracle bit for bit."""
     import torch
     import ter_amd as T
     from hypothesis import given, settings, strategies as st
@@ -157,9 +156,10 @@ def test_quant_int8_kernel(cuda):
 
 
 def run_plan(specs, seed, wgs, with_acc=True):
-    """Build a GemmPlan over `specs`, launch it twice per launch shape and
-    compare every item with the oracle (outputs poisoned between launches).
-    with_acc=False: fp32 outputs only (the kernels' store path for that form)."""
+    """Build a GemmPlan over `specs`, launch it twice and compare every item with
+    the oracle (outputs poisoned between launches), once for each wg_per_cu (it
+    does not change the launch).  with_acc=False: fp32 outputs only (the
+    kernels' store path for that form)."""
     import torch
     import ter_amd as T
     items, refs = [], []
@@ -189,7 +189,7 @@ def run_plan(specs, seed, wgs, with_acc=True):
 
 def test_gemm_plan_mixed(cuda):
     """Many GEMMs in one launch (GemmPlan): ragged shapes, different M per
-    item, unaligned K (byte-wise X staging), launched twice."""
+    item, unaligned K (loads at any address), launched twice."""
     run_plan([(8, 2560, 640), (32, 2560, 2560), (3, 300, 20), (17, 6912, 256), (8, 2048, 512), (1, 64, 16)],
              900, (0, 1))
 
@@ -199,10 +199,8 @@ def test_gemm_plan_mixed(cuda):
     [(256, 512, 64), (140, 300, 20)],
 ], ids=["row_pieces", "bytewise_x"])
 def test_gemm_plan_prefill(cuda, specs):
-    """M above 128: with every X 16-byte aligned (K a multiple of 16) each item
-    is cut into pieces of 128 rows for the LDS-ring kernel (a piece may hold
-    fewer rows); with a byte-wise X in the list the register-staged kernel
-    takes all rows at once."""
+    """M above 128 on the split kernel: pieces of 16 to 64 rows (a piece may hold
+    fewer), with 16-byte aligned X and with rows at any address in the list."""
     run_plan(specs, 500, (0,))
 
 
@@ -211,40 +209,33 @@ def test_gemm_plan_prefill(cuda, specs):
     [(8, 2560, 640), (8, 2560, 2560), (1, 256, 16), (16, 512, 4000), (4, 6912, 2560)],
 ], ids=["bytewise_x", "vector_x"])
 def test_gemm_plan_small_m(cuda, specs):
-    """Small-M plans with a K = 6912 item: 16 rows of it do not fit the
-    streamed kernel's LDS, so these run the LDS-ring kernel (ragged M, K and
-    N, byte-wise and vector X), at several launch shapes."""
+    """Small-M plans with a K = 6912 item on the split kernel: ragged M, K and N,
+    rows at any address and 16-byte aligned."""
     run_plan(specs, 700, (0, 1, 2))
 
 
 @pytest.mark.parametrize("M", [16, 32, 100, 128])
 @pytest.mark.parametrize("with_acc", [True, False], ids=["y_and_acc", "y_only"])
 def test_gemm_plan_list_schedule(cuda, M, with_acc):
-    """LDS-ring plans whose blocks the host deals out largest first: K = 6912
-    blocks (27 units) first, then K = 2560, then many one-unit blocks (K =
-    256) back to back at the end of each workgroup's list, partial blocks at
-    every ragged N, ragged M (100 rows: lanes past the last row store
-    nothing), with and without int32 outputs (fp32 outputs alone take the
-    branch-free store path)."""
+    """Plans of one long, several short and many one-unit GEMMs (K = 6912, 2560,
+    256), whose blocks run longest first; partial blocks at every ragged N,
+    ragged M (100 rows), with and without int32 outputs."""
     run_plan([(M, 6912, 2560), (M, 256, 640), (M, 256, 48), (M, 512, 4000), (M, 256, 1024), (M, 2560, 256),
               (M, 256, 4096)], 1300 + M, (0,), with_acc)
 
 
 @pytest.mark.parametrize("specs", [
-    [(2, 256, 245760)],                    # Ku = 1: 16-strip output buffers, 12-tile chunks, 15 strips per wave
-    [(8, 2560, 12000), (8, 6912, 2560)],   # M = 8 beside K = 6912: 5-strip buffers, 36-tile chunks, ragged last strip
+    [(2, 256, 245760)],                    # one unit of K per block
+    [(8, 2560, 12000), (8, 6912, 2560)],   # M = 8 beside K = 6912, ragged last strip
     [(3, 2560, 6000), (7, 2048, 1000), (16, 512, 4096)],  # ragged M: lanes past the last row store nothing
-    [(2, 256, 1 << 20)],                   # as long as these lists are, the LDS ring takes them (>= 4 blocks per CU)
+    [(2, 256, 1 << 20)],
     [(8, 2560, 262144), (8, 6912, 2560)],
 ], ids=["ku1_long_runs", "m8_bitnet_k", "ragged_m", "ring_ku1", "ring_m8"])
 @pytest.mark.parametrize("with_acc", [True, False], ids=["y_and_acc", "y_only"])
 def test_gemm_stream_chunks(cuda, specs, with_acc):
-    """The streamed kernel (M <= 16 where the X image and the output buffers
-    fit, and the list too short for the LDS ring): at one workgroup per CU each
-    wave's run spans several chunks, so completed strips are buffered in LDS
-    and written between chunks many times per wave; fp32 outputs alone take
-    the branch-free store path.  The last two lists are long enough (at least
-    4 ring blocks per CU on MI355X's 256 CUs) for the LDS ring."""
+    """Long runs of strips at M <= 16: one-unit K, M = 8 beside K = 6912, ragged
+    M, and lists long enough for the LDS ring (the first, fourth and fifth),
+    whose fp32 outputs alone take the branch-free store path."""
     run_plan(specs, 1300, (1,), with_acc)
 
 
@@ -274,8 +265,8 @@ def test_gemm_plan_bitnet_layer(cuda, M):
 
 @pytest.mark.parametrize("M,K,N", [(8, 2560, 640), (32, 2560, 128), (128, 6912, 64), (200, 512, 48)])
 def test_gemm_payload_magnitude(cuda, M, K, N):
-    """{-m, 0, +m} payloads (m = 9841) on every GEMM kernel (streamed M <= 16,
-    LDS ring, pieces of 128 rows) and in a GEMM plan: each row's fp32 output
+    """{-m, 0, +m} payloads (m = 9841) at four row counts and in a GEMM plan (the
+    split kernel; test_gemm_ring_gpu.py has the ring): each row's fp32 output
     is the reference mm_row's float(int64 m * acc) * fl(xs * ws), bit for bit."""
     import torch
     import ter_amd as T

@@ -2,11 +2,13 @@
 activation kind at the last unit count of one compiled bound and the first of
 the next, with the last unit partial, as a single GEMV, as a list whose other
 GEMV is shorter (units past the short K's range are staged nowhere), and as a
-list that shares one activation vector.  Bit for bit."""
+list that reads one activation vector, its weights apart and back to back (the
+shared launch form).  Bit for bit."""
 import numpy as np
 import pytest
 
 from oracle import oracle as O
+from ter_amd._lib import PLAN_SHARED, PLAN_STRIDED
 
 pytestmark = pytest.mark.gpu
 
@@ -60,8 +62,9 @@ def test_strided_bounds(cuda, kind, units):
     act, q, s = problem(kind, K, 11 * K)
     short, qs, ss = problem(kind, 272, 5 * K)
 
-    def check(items, refs):
+    def check(items, refs, shared=False):
         plan = T.Plan(items)
+        assert plan.mode & PLAN_STRIDED and bool(plan.mode & PLAN_SHARED) == shared
         for _ in range(2):
             for it in items:
                 it["y"].fill_(-3)
@@ -81,6 +84,9 @@ def test_strided_bounds(cuda, kind, units):
             T.gemv(W, y=y, **act)
             assert (y.cpu().numpy().view(np.uint32) == refs[-1].view(np.uint32)).all()
     check(items, refs)
+    for it, W in zip(items, T.group_contiguous([it["w"] for it in items])):
+        it["w"] = W
+    check(items, refs, shared=True)
     W, v11 = weights(272, 40, K + 9)
     check([dict(w=W, y=torch.empty(40, dtype=torch.float32, device="cuda"), **short), items[0]],
           [O.gemv_v11(qs, ss, v11, 0.037, 272, 40)[1], refs[0]])

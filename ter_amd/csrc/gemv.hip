@@ -892,7 +892,7 @@ __device__ __forceinline__ void x_prefetch_strided(const GemvDesc& d, XStrided<k
 // a wave-level fence orders them before the loop.  Results are stage_x_vec's
 // bit for bit.  Needs Ku <= max_strided_ku and the fp32 staging (stage32);
 // gs16: fp16 gamma [Ku*256], red: 1024 + 16 floats.
-template <int kKind, int kW, int kU>
+template <int kKind, int kW, int kU, bool kBranch>
 __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrided<kKind, kW, kU>& r, int8_t* lds_x,
                                                  int* usum, float* red, float* xs32, uint16_t* gs16, int u0, int u1,
                                                  bool owner) {
@@ -910,7 +910,7 @@ __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrid
     // of `red`, which its partials overwrite below, gamma to the start of
     // lds_x, which is written after the barriers: a branch per value cuts the
     // loop into blocks, each of which waits for every load in flight, the
-    // first weight batch included.
+    // first weight batch included.  (kBranch: that form all the same.)
     float* const spare = red + (XS::R2 ? V * t : t);
     uint16_t* const spare16 = reinterpret_cast<uint16_t*>(lds_x) + lane;
 #pragma unroll
@@ -931,8 +931,16 @@ __device__ __forceinline__ float stage_x_strided(const GemvDesc& d, const XStrid
             P[e] = __builtin_fmaf(x[j][e], x[j][e], P[e]);  // past K: fma(0, 0, p) = p
             const int i = XS::R2 ? V * t + e + 1024 * j : t + T * j;
             const bool in = i < Ku * kUnitK;  // the staged range
-            *(in ? xs32 + i : spare + e) = x[j][e];
-            *(in ? gs16 + i : spare16) = XS::R2 ? gh : (uint16_t)r.g[j][0];
+            const uint16_t gv = XS::R2 ? gh : (uint16_t)r.g[j][0];
+            if constexpr (kBranch) {
+                if (in) {
+                    xs32[i] = x[j][e];
+                    gs16[i] = gv;
+                }
+            } else {
+                *(in ? xs32 + i : spare + e) = x[j][e];
+                *(in ? gs16 + i : spare16) = gv;
+            }
         }
     }
 #pragma unroll
@@ -1614,7 +1622,11 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
         // skipped the loads in flight are not known and the prologue waits for
         // these too.  With the staging's stores likewise without branches, per
         // Llama token 459 -> 424 us.)
-        load_b(wa);
+        // The widest relu^2 form of a list keeps the branches: 24 loads per thread
+        // before the weights' (K = 8192, N = 2560: 6.2 us without them, 6.0 with;
+        // weights from HBM 7.2, 7.0; the single launch 6.4, 6.6).
+        constexpr bool kBranch = kList && kKind == TER_HIP_X_RELU2_RMS && kU > 28;
+        if (!kBranch || nw > 0) load_b(wa);
         if constexpr (kShared) {
             // the descriptors the outputs need, in flight with the activation
             // and weight loads (left alone the compiler issues them at the
@@ -1637,8 +1649,8 @@ __global__ __launch_bounds__(64 * kW) void gemv_strip_kernel(GemvDesc single, co
             if constexpr (XStrided<kKind, kW, kU>::ABS)
                 act = stage_x_abs_strided<kKind, kW, kU>(d, xst, lds_x, usum, red_s, xs32, u0, u0 + nw, sg == d.strip0);
             else
-                act = stage_x_strided<kKind, kW, kU>(d, xst, lds_x, usum, red_s, xs32, gs16, u0, u0 + nw,
-                                                 sg == d.strip0);
+                act = stage_x_strided<kKind, kW, kU, kBranch>(d, xst, lds_x, usum, red_s, xs32, gs16, u0, u0 + nw,
+                                                              sg == d.strip0);
         } else {
             act = stage_x_vec<kKind>(d, xraw, lds_x, usum, red, xs32, sg == d.strip0);
             __syncthreads();

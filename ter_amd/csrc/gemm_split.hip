@@ -1,7 +1,8 @@
 // gemm_split.hip -- batched packed-trit GEMM for short launches on gfx950
 // MFMA: one GEMM, or a list too short to give the CUs a block each of the
 // LDS-ring kernel (gemm_lds.hip), whose blocks each walk all of K alone; and
-// every GEMM whose X rows are not 16-byte aligned.
+// every GEMM whose X rows are not 16-byte aligned; short single int8 GEMVs as M
+// = 1 (int8_gemv_on_gemm in abi.hip).
 //
 // Same semantics as gemm_lds.hip (cuda/ter_cuda_addonly_batched.cu:117-123):
 // acc[m][j] = sum_k X[m][k] w[k][j] in exact int32, y = float(mag * acc) * (xs[m] * w_scale).
@@ -17,17 +18,18 @@
 // 6912, N = 2560 ten workgroups took 25 us.  With a tile per CU and K split
 // over 4 to 16 waves the launch is a round of loads, a few steps per wave and
 // one LDS exchange; what is left is the launch (about 3 us with its first
-// loads) and each CU's read of its X rows from L2 (R K bytes; 25-40 bytes per
-// clock and CU).  Measured (HIP events, back-to-back launches over 8 weight
-// copies, against the kernels that ran before): M = 8, 2560 x 2560 3.4 us
-// (9.0); M = 64, 2560 x 6912 5.9 us (14.5) and 6912 x 2560 7.3 us (25); M =
-// 256, 2560 x 6912 9.8 us (39, two launches); M = 256, 8192 x 8192 21 us
-// (90); M = 77, 1003 x 1236 (unaligned rows) 3.8 us (57).
+// loads) and each CU's read of its X rows and weights from L2, at 15-28 bytes
+// per clock and CU by the L2's request counters, with the matrix cores busy
+// 7-20% of the time.  Measured in graphs, weights from HBM / cached, the
+// kernels that ran before in parentheses: M = 8, 2560 x 2560 4.9 / 3.3 us (8.6 /
+// 8.1); M = 64, 2560 x 6912 7.3 / 5.9 (13.2 / 12.6) and 6912 x 2560 9.7 / 7.4 (25.7 /
+// 25.3); M = 256, 2560 x 6912 11.8 / 10.9 (39 / 38, two launches); M = 256, 8192 x
+// 8192 25.7 / 24.6 (90 / 89); M = 77, 1003 x 1236 (rows at any address), HIP
+// events, 3.8 us (57).
 //
 // Loads.  X goes through registers to LDS: a load instruction covers 8 rows x
 // 128 bytes, whole cache lines.  (Loading the MFMA A operand straight from
-// memory covers 16 rows x 64 bytes, and each such load cost a CU about 80
-// cycles: 10.8 against 7.3 us at M = 64, K = 6912.)  The weights are gathered
+// memory covers 16 rows x 64 bytes: 10.8 against 7.3 us at M = 64, K = 6912.)  The weights are gathered
 // into the MFMA B operand layout by dword loads (lane = column j + 16 * k
 // group g; one dword = 16 trits), one line per column quad and step.  D steps
 // are in flight in registers; step i + 1 is written to LDS while step i is

@@ -613,7 +613,8 @@ class GemmPlan:
     """Many independent M > 1 GEMMs in one launch.  `items` is a sequence of
     dicts {w: PackedTrits, x: int8 [M][K] tensor, x_scale_dev: fp32 [M]
     tensor, y?: fp32 [M][N], acc?: int32 [M][N], y16?: fp16 [M][N],
-    resid?: fp32 [M][N]}."""
+    resid?: fp32 [M][N]}.  The kernel and its launch shape follow from the
+    list's shapes; wg_per_cu is accepted, as Plan's, and changes nothing."""
 
     def __init__(self, items: Sequence[dict], wg_per_cu: int = 0):
         n = len(items)

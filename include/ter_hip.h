@@ -100,7 +100,9 @@ extern "C" {
  * 16 output columns x 256 input rows, 2 bits per trit, stored as u = w + 1
  * (dword 4L+j of a tile holds column 4(L/16)+j of the tile's strip over rows
  * 16(L%16)+e, e = 4f+b at bits 8b+2f), followed by `N` 64-bit fix-up slots
- * (`fix`, zero at rest) used to combine split column strips.  The whole
+ * (`fix`, zero at rest) used to combine split column strips: GEMV launches of
+ * one weight that split strips between workgroups must not run at the same
+ * time.  The whole
  * buffer is `ter_hip_wpk_bytes(K, N)` bytes of device memory owned by the
  * caller.  `scale` is the per-tensor weight scale (Wt.scale).  A ternary
  * payload {-m,0,+m} is stored as trits {-1,0,+1} with m in `mag` (1 for

@@ -249,29 +249,32 @@ bool strip_mode_ok(long long total_tiles, long long total_strips, int cus) {
     return total_tiles < (long long)cus * kGemvWgPerCu * kSmallPlanTilesPerWg && total_strips <= (long long)cus * 4;
 }
 
-// Whether a single GEMV on int8 rows runs the GEMM kernels at M = 1 (which
-// need no prologue; fifteen of an MFMA's sixteen rows are padding) instead of
-// the GEMV kernels with the int8 prologue.  In graphs, GEMM against GEMV, over
-// weights from HBM (over cached ones):
-//   vec rows, strip mode: 256 x 640 3.3 against 3.7 us (2.6, 2.9), 1024 x 4096
-//     3.75, 3.83 (2.8, 3.05), but 1024 x 8192 4.35, 4.23 (3.25, 3.4), 2560 x 640
-//     4.5, 4.0 (3.2, 3.2), 6912 x 2560 6.2, 4.9: GEMM for the shortest only.
-//   vec rows past strip mode (stream-K): at most two strips per CU 8192 x 8192
-//     8.4, 8.15 (6.3, 7.1), 12288 x 8192 9.9, 10.0 (7.3, 8.8), but 16384 x 8192
-//     12.1, 11.5; up to four strips per CU 6912 x 12288 11.0, 9.0; beyond (ring
-//     kernel and its device scales) 3072 x 24576 8.1, 8.9 and 4096 x 24576 11.4,
-//     9.8; 2048 x 32768 8.1, 8.1 and 2560 x 32768 9.5, 8.9; 2048 x 128256 14.1,
-//     16.6, 4096 x 128256 27.0, 27.3 and 8192 x 128256 50.9, 46.2.
-//   other rows (the general prologue): at most two strips per CU 3501 x 8192
-//     7.4, 8.0 (5.4, 7.2), but 4001 x 8192 7.6, 7.0; up to four 1003 x 16384
-//     6.6, 7.4, but 1501 x 16384 8.1, 7.7; more 255 x 32768 8.3, 7.3.
-bool int8_gemv_on_gemm(long long strips, int Ku, bool vec, bool dev_scale, int cus) {
+// The kernel of a single GEMV on int8 rows: the GEMM kernels at M = 1 (which
+// need no prologue; fifteen of an MFMA's sixteen rows are padding), or the strip
+// or stream-K kernel with the int8 prologue (vec: 16-byte rows) or the general
+// one.  In graphs, weights from HBM (cached):
+//   vec, GEMM against strip: 256 x 640 3.3, 3.7 us (2.6, 2.9), 1024 x 4096 3.75,
+//     3.83 (2.8, 3.05), but 1024 x 8192 4.35, 4.23 (3.25, 3.4), 2560 x 640 4.5, 4.0
+//     (3.2, 3.2), 6912 x 2560 6.2, 5.0; on more than four strips per CU 512 x 32768
+//     4.6, 5.0, but 1024 x 24576 5.45, 5.1 and 2048 x 24576 7.0, 6.5; from eight or
+//     ten on 2560 x 40960 8.2, 8.6, 4096 x 40960 10.9, 10.7, 6912 x 49152 16.5, 17.9,
+//     2048 x 128256 14.1, 15.4, 8192 x 128256 50.9, 46.4 (this one goes to the
+//     slower).  A host scale rules the ring kernel out, which those need.
+//   vec, strip against stream-K: 6912 x 12288 8.1, 9.1, 8192 x 32768 14.4, 17.4,
+//     12288 x 16384 12.0, 13.0; past 48 units of K and two strips per CU 16384 x
+//     10240 13.5, 12.3 and 16384 x 16384 15.9, 17.7 (GEMM 20.5).
+//   other rows, GEMM against the general prologue: at most two strips per CU
+//     3501 x 8192 7.4, 8.0 (5.4, 7.2), but 4001 x 8192 7.6, 7.0; up to four 1003 x
+//     16384 6.6, 7.4, but 1501 x 16384 8.1, 7.7; more 255 x 32768 8.3, 7.3.
+enum class Int8Route { gemm, strip, stream };
+Int8Route int8_gemv_route(long long strips, int Ku, bool vec, bool dev_scale, int cus) {
     const long long rounds = (strips + cus - 1) / cus;
-    if (!vec) return rounds <= 2 ? Ku <= 14 : rounds <= 4 && Ku <= 4;
-    if (strip_mode_ok(strips * Ku, strips, cus)) return Ku * rounds <= 4;
-    if (rounds <= 2) return Ku <= 48;
-    if (rounds <= 4 || !dev_scale) return false;
-    return Ku <= (strips >= 16LL * cus ? 16 : (strips >= 8LL * cus ? 8 : 12));
+    if (!vec) {
+        if (rounds <= 2 ? Ku <= 14 : rounds <= 4 && Ku <= 4) return Int8Route::gemm;
+        return strip_mode_ok(strips * Ku, strips, cus) ? Int8Route::strip : Int8Route::stream;
+    }
+    if (Ku * rounds <= 4 || (dev_scale && rounds > (Ku <= 2 ? 4 : (Ku <= 10 || Ku > 48 ? 8 : 10)))) return Int8Route::gemm;
+    return rounds <= 2 || (rounds <= 10 && Ku <= 48) ? Int8Route::strip : Int8Route::stream;
 }
 
 int gemv_vec_kind(const ter_hip_gemv_item_t* items, int n) {
@@ -282,21 +285,13 @@ int gemv_vec_kind(const ter_hip_gemv_item_t* items, int n) {
 
 // The workgroups of a launch in strip mode: one per strip up to one per CU (two
 // for int8 inputs, which have no prologue to repeat).
-int pick_strip_mode(long long total_tiles, long long total_strips, bool prologue, bool* strip_mode, int* n_wg) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    const int cus = device_cu_count(dev);
-    if (cus <= 0) return fail(TER_HIP_ERR_HIP, "cannot query CU count");
-    *strip_mode = strip_mode_ok(total_tiles, total_strips, cus);
-    if (!*strip_mode) return TER_HIP_OK;
+int strip_mode_wg(long long total_strips, bool prologue, int cus) {
     long long g = (long long)cus * (prologue ? 1 : kGemvWgPerCu);
     if (g > total_strips) g = total_strips;
     const long long min_g = (total_strips + kStripModeMaxStrips - 1) / kStripModeMaxStrips;
     if (g < min_g) g = min_g;
     if (g < 1) g = 1;
-    *n_wg = (int)g;
-    return TER_HIP_OK;
+    return (int)g;
 }
 
 int pick_wg(long long total_tiles, int wg_per_cu, int lds_bytes, bool prologue, int vec_kind, int* n_wg) {
@@ -1052,8 +1047,13 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
     rc = current_cu_count(&cus);
     if (rc) return rc;
     const int vec_kind = act_vec_kind(*x, w->K);
-    if (x->kind == TER_HIP_X_I8 && !out->resid16 && !out->silu &&
-        int8_gemv_on_gemm(strips_of(w->N), units_of(w->K), vec_kind >= 0, x->scale_dev != nullptr, cus)) {
+    bool strip_mode = strip_mode_ok(total, strips_of(w->N), cus);
+    Int8Route route = Int8Route::stream;
+    if (x->kind == TER_HIP_X_I8) {
+        route = int8_gemv_route(strips_of(w->N), units_of(w->K), vec_kind >= 0, x->scale_dev != nullptr, cus);
+        strip_mode = route == Int8Route::strip || (route == Int8Route::gemm && strip_mode);
+    }
+    if (route == Int8Route::gemm && !out->resid16 && !out->silu) {
         GemmDesc gd = make_gemm_desc(w, static_cast<const int8_t*>(x->data), x->scale_dev, 1, *out);
         gd.x_scale = x->scale;
         return run_gemm(gd, *out, static_cast<hipStream_t>(stream));
@@ -1067,10 +1067,8 @@ int ter_hip_gemv_out(const ter_hip_wpk_t* w, const ter_hip_act_t* x, const ter_h
     // 5.6, fp16 absmax 5.9 -> 3.9 against the general one), and strip mode for
     // small GEMVs (whole strips per workgroup, the waves' partials added in
     // LDS, no fix-up slots)
-    bool strip_mode = false;
-    rc = pick_strip_mode(total, d.n_strips, prologue, &strip_mode, &n_wg);
-    if (rc) return rc;
     if (strip_mode) {
+        n_wg = strip_mode_wg(d.n_strips, prologue, cus);
         const bool strided = gemv_strided_ok(vec_kind, w->K, d.stage32 != 0);
         const int waves = strided ? gemv_strided_waves(vec_kind) : kGemvWaves;
         const int part_off = (gemv_strip_part_off(w->K, d.stage32 != 0) + 15) / 16 * 16;
@@ -1316,8 +1314,11 @@ int ter_hip_plan_create(ter_hip_plan_t** plan, const ter_hip_gemv_item_t* items,
     bool strip_mode = false;
     int part_off = 0;
     if (wg_per_cu <= 0) {
-        rc = pick_strip_mode(tile, strips, prologue, &strip_mode, &n_wg);
+        int cus = 0;
+        rc = current_cu_count(&cus);
         if (rc) return rc;
+        strip_mode = strip_mode_ok(tile, strips, cus);
+        if (strip_mode) n_wg = strip_mode_wg(strips, prologue, cus);
     }
     bool strided = false;
     if (strip_mode) {

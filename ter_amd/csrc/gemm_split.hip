@@ -2,7 +2,7 @@
 // MFMA: one GEMM, or a list too short to give the CUs a block each of the
 // LDS-ring kernel (gemm_lds.hip), whose blocks each walk all of K alone; and
 // every GEMM whose X rows are not 16-byte aligned; short single int8 GEMVs as M
-// = 1 (int8_gemv_on_gemm in abi.hip).
+// = 1 (int8_gemv_route in abi.hip).
 //
 // Same semantics as gemm_lds.hip (cuda/ter_cuda_addonly_batched.cu:117-123):
 // acc[m][j] = sum_k X[m][k] w[k][j] in exact int32, y = float(mag * acc) * (xs[m] * w_scale).

@@ -90,8 +90,8 @@ def test_gemv_single_int8(cuda, K, N, shift, scale):
 
 
 # both sides of the lines between the GEMM kernels, strip mode and stream-K (256 CUs)
-ROUTES = [(1024, 4096), (1024, 4112), (1040, 64), (8192, 8176), (8192, 8192), (12288, 5472), (12304, 5472),
-          (1024, 16400), (3088, 16400), (2064, 32768), (3583, 8192), (3585, 64), (1025, 8208)]
+ROUTES = [(1024, 4096), (1024, 4112), (1040, 64), (8192, 8192), (12288, 8208), (12304, 8208), (512, 16400),
+          (528, 16400), (3088, 16400), (2064, 32768), (2064, 32784), (2816, 40960), (3583, 8192), (3585, 64), (1025, 8208)]
 
 
 @pytest.mark.parametrize("scale", ["device", "host"])

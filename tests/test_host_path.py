@@ -134,14 +134,14 @@ VEC_STREAM, STREAM, SPLIT, RING = "gemv_t16_kernel<false, 0>", "gemv_t16_kernel<
 
 
 @pytest.mark.parametrize("K,N,shift,dev_scale,kernel", [
-    # 16-byte aligned rows, strip mode: the GEMM kernels for the shortest only
+    # 16-byte aligned rows: the GEMM kernels for the shortest, strip mode, stream-K past 48 units and two strips per CU
     (1024, 4096, 0, 1, SPLIT), (1024, 4096, 0, 0, SPLIT), (1024, 4112, 0, 1, VEC_STRIP), (1040, 64, 0, 1, VEC_STRIP),
-    (2560, 640, 0, 1, VEC_STRIP), (2560, 640, 0, 0, VEC_STRIP), (32768, 2048, 0, 1, VEC_STREAM),
-    # past it: up to two strips per CU, up to four, eight, sixteen and more
-    (8192, 8176, 0, 1, VEC_STRIP), (8192, 8192, 0, 1, SPLIT), (12288, 5472, 0, 0, SPLIT), (12304, 5472, 0, 1, VEC_STREAM),
-    (4096, 16384, 0, 1, VEC_STREAM), (3072, 16400, 0, 0, VEC_STREAM), (3088, 16400, 0, 1, VEC_STREAM),
-    (2048, 32768, 0, 1, RING), (2064, 32768, 0, 1, VEC_STREAM), (4096, 65536, 0, 1, RING), (4096, 65536, 0, 0, VEC_STREAM),
-    (4112, 65536, 0, 1, VEC_STREAM),
+    (2560, 640, 0, 1, VEC_STRIP), (2560, 640, 0, 0, VEC_STRIP), (32768, 8192, 0, 1, VEC_STRIP),
+    (12288, 8208, 0, 1, VEC_STRIP), (12304, 8208, 0, 1, VEC_STREAM), (12288, 40960, 0, 0, VEC_STRIP),
+    # from four, eight and ten strips per CU on
+    (512, 16400, 0, 1, RING), (512, 16400, 0, 0, VEC_STRIP), (528, 16400, 0, 1, VEC_STRIP), (4096, 40960, 0, 1, VEC_STRIP),
+    (2560, 32768, 0, 1, VEC_STRIP), (2560, 32784, 0, 1, RING), (12304, 32768, 0, 1, VEC_STREAM), (12304, 32784, 0, 1, RING),
+    (4096, 40976, 0, 1, RING), (4096, 40976, 0, 0, VEC_STREAM), (8192, 65536, 0, 1, RING),
     # other rows
     (3583, 8192, 0, 1, SPLIT), (3585, 64, 0, 1, STRIP), (3584, 8192, 1, 0, SPLIT), (3600, 64, 1, 1, STRIP),
     (1023, 16384, 0, 1, SPLIT), (1025, 8208, 0, 1, STRIP), (1023, 16400, 0, 1, STREAM), (15, 8, 0, 1, SPLIT),

@@ -482,11 +482,13 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int hip_fail(hipError_t e, const char* what);
 
 int device_cu_count(int device);
-// Raises the limit on a launch's dynamic LDS (64 KiB by default) for some
-// kernels, once for each device that they run on; failures are not kept.
+// Raises the limit on a launch's dynamic LDS (64 KiB by default, enough for most
+// launches, which then ask for nothing) for some kernels, once for each device
+// that they run on; failures are not kept.
 class LdsLimit {
 public:
     hipError_t allow(int bytes, std::initializer_list<const void*> kernels) {
+        if (bytes <= 64 * 1024) return hipSuccess;
         int dev = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return e;
